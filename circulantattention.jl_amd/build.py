@@ -26,6 +26,7 @@ SOURCES = ["api.cpp", "unfused.hip", "apply_rb.hip", "fused.hip", "fused_fwd.hip
            "fused2h2_fwd.hip", "fused2h2_bwdq.hip", "fused2h2_bwdkv.hip", "fused1h_fwd.hip",
            "fused1h_bwdq.hip", "fused1h_bwdkv.hip", "fused1h2_fwd.hip", "fused1h2_bwdq.hip",
            "fused1h2_bwdkv.hip", "fused_wide.hip",
+           *(f"fused_stream{n}_{m}.hip" for n in (1, 2, 3, 4) for m in ("fwd", "bwdq", "bwdkv")),
            "batch_ops.hip"]
 FLAGS = [
     f"--offload-arch={ARCH}",

@@ -85,6 +85,14 @@ __host__ __device__ __forceinline__ void banded_tile(int t, int tiles_h, int til
     }
 }
 
+// ln(2^m l) - d, rounded once: every probability of the row that the backward
+// forms carries this number's error
+__device__ __forceinline__ float lse_of(float m, float l, float d) {
+    const int e = __builtin_amdgcn_frexp_expf(l);
+    const double l2 = (double)m + (double)e + (double)__builtin_amdgcn_logf(__builtin_amdgcn_frexp_mantf(l));
+    return (float)(l2 * 0.69314718055994530942 - (double)d);
+}
+
 // Geometry of one problem: nsp spatial dims, N1 (fastest) and N2 (1 for 1D),
 // window ws along each spatial dim.
 struct Geom {

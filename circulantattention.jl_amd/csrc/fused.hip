@@ -3,6 +3,7 @@
 #include "fused2d_impl.h"
 #include "fused2h_impl.h"
 #include "fused_impl.h"
+#include "fused_stream_impl.h"
 #include "fused_wide_impl.h"
 
 namespace circatt {
@@ -190,7 +191,7 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
         if (mode == MODE_FWD) e = launch_f2h2_fwd(pr.g.p, cplx, dist, a, cus, s);
         if (mode == MODE_BWDQ) e = launch_f2h2_bwdq(pr.g.p, cplx, dist, a, cus, s);
         if (mode == MODE_BWDKV) e = launch_f2h2_bwdkv(pr.g.p, cplx, dist, a, cus, s);
-        if (e != hipErrorNotSupported) return e;
+        return e;  // (windows past 11: launch_stream)
     }
     switch (mode) {
     case MODE_FWD: return launch_f2d_fwd(pr.g.p, nt, cplx, dist, a, cus, s);
@@ -200,9 +201,61 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
     }
 }
 
+// Streamed split-half kernels (fused_stream_impl.h): any window, up to 64 real
+// components per head; hipErrorNotSupported otherwise.  Buffer offsets are 32
+// bits, and channels-last components are loaded four at a time.
+hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
+    const int ncr = pr.dh * pr.ncomp;
+    const int64_t all = (int64_t)pr.nheads * ncr;
+    if (mode == MODE_SIM || math_mode() != CIRCATT_MATH_SPLIT_F16 || ncr > 64 || pr.nunits > INT32_MAX ||
+        pr.g.p < 1 || pr.g.P * (pr.cl ? all : ncr) * 4 >= (int64_t)fst::kMaxBytes || (pr.cl && ncr % 4 != 0))
+        return hipErrorNotSupported;
+    // Windows of fewer keys stay on the Float32 products: there the halves'
+    // error (2^-24 to 2^-23 of a product) is the larger (measured against 64
+    // bits on N(0,1) data, errors of y at 8, 16 components: 1.34 x at ws 3,
+    // 1.13 x at ws 9, below 1 x from ws 23; 48, 64: 1.2 x at ws 3, at most 1 x
+    // from ws 5; gradients, whose probabilities this family rounds less, below
+    // 1 x from ws 7 at 8 components).
+    const int nt = (ncr + 15) / 16;
+    static constexpr int kMinFwd[4] = {400, 49, 25, 15}, kMinBwd[4] = {49, 31, 25, 15};
+    if (pr.g.K < (mode == MODE_FWD ? kMinFwd : kMinBwd)[nt - 1]) return hipErrorNotSupported;
+    fst::Args a{};
+    a.q = pr.q; a.k = pr.k; a.v = pr.v; a.y = pr.y; a.dy = pr.dy; a.lse = pr.lse;
+    a.yout = pr.yout; a.lse_out = pr.lse_out; a.dq = pr.dq; a.dk = pr.dk; a.dv = pr.dv;
+    a.dbuf = pr.dbuf;
+    a.n1 = pr.g.n1;
+    a.n2 = pr.g.n2;
+    a.P = (int)pr.g.P;
+    a.ncr = ncr;
+    a.ncrall = (int)all;
+    a.lay = pr.cl ? fst::LAST : pr.ncomp == 2 ? fst::PLANAR_C : fst::PLANAR;
+    a.nheads = pr.nheads;
+    a.unit_stride = (int)(pr.g.P * ncr);
+    a.scale = pr.scale;
+    a.c2 = pr.scale * kLog2e;
+    a.p = pr.g.p;
+    a.pe = 1;
+    while (a.pe < 10 && (1 << (a.pe + 1)) < pr.g.K) ++a.pe;
+    a.fine = pr.g.K < 64;
+    const bool one = pr.g.nsp == 1, dist = pr.kind == 1;
+    const int nu = (int)pr.nunits, cus = device_cus();
+#define CIRCATT_FST_MODE(M)                                        \
+    switch (nt) {                                                  \
+    case 1: return launch_fst_##M##_1(one, dist, a, nu, cus, s);     \
+    case 2: return launch_fst_##M##_2(one, dist, a, nu, cus, s);     \
+    case 3: return launch_fst_##M##_3(one, dist, a, nu, cus, s);     \
+    default: return launch_fst_##M##_4(one, dist, a, nu, cus, s);    \
+    }
+    if (mode == MODE_FWD) CIRCATT_FST_MODE(fwd)
+    if (mode == MODE_BWDQ) CIRCATT_FST_MODE(bwdq)
+    CIRCATT_FST_MODE(bwdkv)
+#undef CIRCATT_FST_MODE
+}
+
 hipError_t launch_fused(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
     if (mode != MODE_SIM) {
         hipError_t e = launch_f2d(mode, pr, s);
+        if (e == hipErrorNotSupported) e = launch_stream(mode, pr, s);
         if (e != hipErrorNotSupported) return e;
     }
     Plan pl = make_plan(mode, pr);

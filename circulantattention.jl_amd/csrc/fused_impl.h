@@ -700,8 +700,7 @@ __global__ __launch_bounds__(256, 2) void fused_kernel(FArgs a) {
                                 yb[comp_index(a, rpix, comp)] = (acc[0][t][r] + acc[1][t][r]) * inv;
                         }
                     if (g == 0)
-                        a.lse_out[soff + rpix] =
-                            (m + log2f(l)) * kLn2 - (DIST ? 0.5f * sq * a.scale : 0.f);
+                        a.lse_out[soff + rpix] = lse_of(m, l, DIST ? 0.5f * sq * a.scale : 0.f);
                 }
             } else if constexpr (MODE == MODE_BWDQ) {
                 const float rs = DIST ? xsum16_32(corr) : 0.f;

@@ -1,0 +1,9 @@
+// Instantiations of the streamed split-half kernels, forward, up to 32 real
+// components per head (fused_stream_impl.h).
+#include "fused_stream_impl.h"
+
+namespace circatt {
+
+CIRCATT_FST_DEF(fwd, fst::FWD, 2)
+
+}  // namespace circatt

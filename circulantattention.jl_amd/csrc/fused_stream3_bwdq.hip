@@ -1,0 +1,9 @@
+// Instantiations of the streamed split-half kernels, query-centric, up to 48 real
+// components per head (fused_stream_impl.h).
+#include "fused_stream_impl.h"
+
+namespace circatt {
+
+CIRCATT_FST_DEF(bwdq, fst::BWDQ, 3)
+
+}  // namespace circatt
