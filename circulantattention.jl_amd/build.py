@@ -20,7 +20,7 @@ INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
-SOURCES = ["api.cpp", "unfused.hip", "apply_rb.hip", "apply_mx.hip", "fused.hip", "fused_fwd.hip", "fused_sim.hip",
+SOURCES = ["api.cpp", "unfused.hip", "apply_rb.hip", "apply_mx.hip", "sim_mx.hip", "fused.hip", "fused_fwd.hip", "fused_sim.hip",
            "fused_bwdq.hip", "fused_bwdkv.hip", "fused2d_fwd.hip", "fused2d_bwdq.hip",
            "fused2d_bwdkv.hip", "fused2h_fwd.hip", "fused2h_bwdq.hip", "fused2h_bwdkv.hip",
            "fused2h2_fwd.hip", "fused2h2_bwdq.hip", "fused2h2_bwdkv.hip", "fused1h_fwd.hip",

@@ -49,6 +49,10 @@ hipError_t launch_apply_mx(bool trans, bool corr, int ncomp, const Geom &g, int 
                            const float *nz, const float *x, const float *z, float *y, hipStream_t s);
 hipError_t launch_apply_mx_pair(bool corr, int ncomp, const Geom &g, int C, int64_t nb, float scale, const float *nz,
                                 const float *x, const float *y, float *dx, float *dy, hipStream_t s);
+// Similarity in 2D from scores held in registers (sim_mx.hip).
+bool sim_mx_supported(bool dist, const Geom &g, int C, int ncomp, int64_t nb);
+hipError_t launch_sim_mx(bool dist, int ncomp, const Geom &g, int C, int64_t nb, float scale, const float *x,
+                         const float *y, float *nz, hipStream_t s);
 // Similarity for windows of any odd width in 1D and 2D (sub-row tasks).
 bool sim_wide_supported(const Geom &g, int C, int ncomp, int64_t nb);
 hipError_t launch_sim_wide(bool dist, int ncomp, const Geom &g, int C, int64_t nb, float scale,
