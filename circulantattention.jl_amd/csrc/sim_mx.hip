@@ -14,7 +14,8 @@
 //
 // What bounds it: dot products by issue (matrix cores a third of the time, the
 // vector instructions of staging and of the rows' assembly a fifth), differences
-// by LDS: a 16-byte read for 8 vector instructions.  200x120, window 23, 32
+// by LDS: a 16-byte read for 8 vector instructions, or 16 where a wavefront
+// takes two query blocks.  200x120, window 23, 32
 // components: 171 -> 48 us, Distance 213 -> 73 us (51 MB of scores, 10 us at the
 // rate of a large copy).
 #include <algorithm>
@@ -75,7 +76,7 @@ __device__ __forceinline__ int wrap(int v, int n) {
     return v - (v >= n ? n : 0);
 }
 
-template <int NK, int CB, bool DIST, bool CPLX>
+template <int NK, int CB, int QH, bool DIST, bool CPLX>
 __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
     const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
     if ((blockIdx.x >> 3) >= a.per_xcd || item >= a.nitems) return;
@@ -92,22 +93,28 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
     const int it = fdiv(item, a.div_strip), strip = item - it * a.nstrip;
     const int unit = fdiv(it, a.div_tiles), tile = it - unit * (a.tiles_h * a.tiles_w);
     const int tw = fdiv(tile, a.div_th);
-    const int h0 = (tile - tw * a.tiles_h) * 4 * kNW, w0 = tw * 4 * kNW;
+    const int h0 = (tile - tw * a.tiles_h) * 4 * QH * kNW, w0 = tw * 4 * kNW;
     const int b0 = strip * CB;  // first block column
     const int64_t xo = (int64_t)unit * a.P * a.ncr;
     const i4v ry = dma_rsrc(a.y + xo, a.P * a.ncr * 4);
     const auto ryb = rsrc(a.y + xo, a.P * a.ncr * 4);
     const auto rxb = rsrc(a.x + xo, a.P * a.ncr * 4);
 
-    const int hw = h0 + 4 * wh, wc = w0 + 4 * ww;  // the wavefront's first pixel
-    const int rh = hw + jr, rw = wc + jc;
-    const int rpix = rh < a.n1 && rw < a.n2 ? rh + a.n1 * rw : 0;
-    // byte offset of component k of the query, past the buffer from ncr on
-    auto qoff = [&](int k) { return k < a.ncr ? ((CPLX ? 2 * a.P * (k >> 1) + (k & 1) : a.P * k) + PF * rpix) * 4 : kOut; };
-
-    f4 acc[NK * CB];
+    const int hw = h0 + 4 * QH * wh, wc = w0 + 4 * ww;  // the wavefront's first pixel
+    const int rh = hw + jr, rw = wc + jc;               // the lane's query, of the first block
+    int rpix[QH];
 #pragma unroll
-    for (int i = 0; i < NK * CB; ++i) acc[i] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < QH; ++b) rpix[b] = rh + 4 * b < a.n1 && rw < a.n2 ? rh + 4 * b + a.n1 * rw : 0;
+    // byte offset of component k of the query, past the buffer from ncr on
+    auto qoff = [&](int b, int k) {
+        return k < a.ncr ? ((CPLX ? 2 * a.P * (k >> 1) + (k & 1) : a.P * k) + PF * rpix[b]) * 4 : kOut;
+    };
+
+    f4 acc[QH][NK * CB];
+#pragma unroll
+    for (int b = 0; b < QH; ++b)
+#pragma unroll
+        for (int i = 0; i < NK * CB; ++i) acc[b][i] = f4{0.f, 0.f, 0.f, 0.f};
 
     for (int c0 = 0; c0 < a.ncr; c0 += 16) {
         if (c0 > 0) __syncthreads();  // the previous components' reads are done
@@ -148,40 +155,51 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
             }
         }
         const int nc = min(16, a.ncr - c0);
-        float q = load(rxb, qoff(c0 + (DIST ? 0 : g)));
+        float q[QH];
+#pragma unroll
+        for (int b = 0; b < QH; ++b) q[b] = load(rxb, qoff(b, c0 + (DIST ? 0 : g)));
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();  // planes staged
         if constexpr (DIST) {
             // key rows 0 .. 3 of block column bc's column g
-            const float *const kb = lds + (4 * wh + a.cr * (4 * ww + g)) * PF;
+            const float *const kb = lds + (4 * QH * wh + a.cr * (4 * ww + g)) * PF;
             for (int k = 0; k < nc; k += PF) {
-                const float qn = load(rxb, qoff(c0 + min(k + PF, nc - 1)));
-                const float qi = CPLX ? load(rxb, qoff(c0 + k + 1)) : 0.f;
+                float qn[QH], qi[QH];
+#pragma unroll
+                for (int b = 0; b < QH; ++b) {
+                    qn[b] = load(rxb, qoff(b, c0 + min(k + PF, nc - 1)));
+                    if constexpr (CPLX) qi[b] = load(rxb, qoff(b, c0 + k + 1));
+                }
                 const float *const kp = kb + k / PF * a.pl;
 #pragma unroll
                 for (int bc = 0; bc < CB; ++bc)
 #pragma unroll
-                    for (int br = 0; br < NK; ++br) {
+                    for (int br = 0; br < NK + QH - 1; ++br) {
                         const float *const kq = kp + 4 * bc * a.cr * PF + 4 * br * PF;
-                        f4 &s = acc[bc * NK + br];
                         const f4 lo = *reinterpret_cast<const f4 *>(kq);
+                        f4 re = lo, im;
                         if constexpr (CPLX) {
                             const f4 hi = *reinterpret_cast<const f4 *>(kq + 4);
-                            const f4 re = f4{lo[0], lo[2], hi[0], hi[2]}, im = f4{lo[1], lo[3], hi[1], hi[3]};
+                            re = f4{lo[0], lo[2], hi[0], hi[2]};
+                            im = f4{lo[1], lo[3], hi[1], hi[3]};
+                        }
+#pragma unroll
+                        for (int b = 0; b < QH; ++b) {  // (query block b meets its block row br - b)
+                            if (br - b < 0 || br - b >= NK) continue;
+                            f4 &s = acc[b][bc * NK + br - b];
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
-                                const float d = q - re[r], e = qi - im[r];
-                                s[r] = __builtin_fmaf(e, e, __builtin_fmaf(d, d, s[r]));
-                            }
-                        } else {
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const float d = q - lo[r];
+                                const float d = q[b] - re[r];
                                 s[r] = __builtin_fmaf(d, d, s[r]);
+                                if constexpr (CPLX) {
+                                    const float e = qi[b] - im[r];
+                                    s[r] = __builtin_fmaf(e, e, s[r]);
+                                }
                             }
                         }
                     }
-                q = qn;
+#pragma unroll
+                for (int b = 0; b < QH; ++b) q[b] = qn[b];
             }
         } else {
             // key (row j & 3, column j >> 2) of a block, component 4 s + g
@@ -194,14 +212,14 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
                     for (int br = 0; br < NK; ++br) {
                         float kv = kp[4 * bc * a.cr * PF + 4 * br * PF];
                         if (part && 4 * s + g >= nc) kv = 0.f;
-                        acc[bc * NK + br] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, q, acc[bc * NK + br], 0, 0, 0);
+                        acc[0][bc * NK + br] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv, q[0], acc[0][bc * NK + br], 0, 0, 0);
                     }
             };
             const int full = nc >> 2;
             for (int s = 0; s < full; ++s) {
-                const float qn = load(rxb, qoff(c0 + 4 * (s + 1) + g));
+                const float qn = load(rxb, qoff(0, c0 + 4 * (s + 1) + g));
                 step(s, false);
-                q = qn;
+                q[0] = qn;
             }
             if (nc & 3) step(full, true);
         }
@@ -214,27 +232,6 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
     // to the wrap.
     float *const out = lds + wv * a.region;
     const float sc = DIST ? -0.5f * a.scale : a.scale;
-    {
-        const int s1 = slot_shift(min(rh, a.n1 - 1) + 1, a.n1, a.p);  // (rows past the image: any slots)
-        const int u0 = max(4 * b0 - jc, 0);
-        int col[CB];
-#pragma unroll
-        for (int bc = 0; bc < CB; ++bc) {
-            const int u2 = 4 * (b0 + bc) + g - jc;
-            col[bc] = u2 >= 0 && u2 <= 2 * a.p ? j * a.seg + (u2 - u0) * a.ws : 1 << 24;
-        }
-        const int dump = 16 * a.seg;
-#pragma unroll
-        for (int br = 0; br < NK; ++br)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int u1 = 4 * br + r - jr;
-                const int m1 = u1 >= 0 && u1 <= 2 * a.p ? wrap(u1 + s1, a.ws) : 1 << 24;
-#pragma unroll
-                for (int bc = 0; bc < CB; ++bc) out[min(col[bc] + m1, dump)] = acc[bc * NK + br][r] * sc;
-            }
-    }
-    // (LDS operations of a wavefront are in order)
     float *const nz = a.nz + (int64_t)unit * a.P * a.K;
     auto copy = [&](const float *src, float *dst, int n) __attribute__((always_inline)) {
         for (int e = 4 * lane; e < n; e += 256) {
@@ -245,21 +242,44 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
             }
         }
     };
-    const int nr = min(4, a.n1 - hw);  // rows of the image
-    for (int c = 0; c < 4; ++c) {
-        if (wc + c >= a.n2 || nr <= 0) break;
-        float *const row = nz + (int64_t)(hw + a.n1 * (wc + c)) * a.K;
-        const int s2 = slot_shift(wc + c + 1, a.n2, a.p);
-        const int u0 = max(4 * b0 - c, 0), u1 = min(4 * (b0 + CB) - c, a.ws);  // window columns [u0, u1)
-        if (u1 <= u0) continue;
-        const int m0 = wrap(u0 + s2, a.ws), n0 = min(u1 - u0, a.ws - m0), n1 = u1 - u0 - n0;
-        if (a.seg == a.K && n1 == 0) {  // whole rows, one after the other
-            copy(out + 4 * c * a.seg, row, nr * a.K);
-        } else {
-            for (int r = 0; r < nr; ++r) {
-                const float *const src = out + (4 * c + r) * a.seg;
-                copy(src, row + r * a.K + m0 * a.ws, n0 * a.ws);
-                if (n1 > 0) copy(src + n0 * a.ws, row + r * a.K, n1 * a.ws);
+#pragma unroll
+    for (int b = 0; b < QH; ++b) {  // (LDS operations of a wavefront are in order)
+        {
+            const int s1 = slot_shift(min(rh + 4 * b, a.n1 - 1) + 1, a.n1, a.p);  // (rows past the image: any slots)
+            const int u0 = max(4 * b0 - jc, 0);
+            int col[CB];
+#pragma unroll
+            for (int bc = 0; bc < CB; ++bc) {
+                const int u2 = 4 * (b0 + bc) + g - jc;
+                col[bc] = u2 >= 0 && u2 <= 2 * a.p ? j * a.seg + (u2 - u0) * a.ws : 1 << 24;
+            }
+            const int dump = 16 * a.seg;
+#pragma unroll
+            for (int br = 0; br < NK; ++br)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int u1 = 4 * br + r - jr;
+                    const int m1 = u1 >= 0 && u1 <= 2 * a.p ? wrap(u1 + s1, a.ws) : 1 << 24;
+#pragma unroll
+                    for (int bc = 0; bc < CB; ++bc) out[min(col[bc] + m1, dump)] = acc[b][bc * NK + br][r] * sc;
+                }
+        }
+        const int nr = min(4, a.n1 - hw - 4 * b);  // rows of the image
+        for (int c = 0; c < 4; ++c) {
+            if (wc + c >= a.n2 || nr <= 0) break;
+            float *const row = nz + (int64_t)(hw + 4 * b + a.n1 * (wc + c)) * a.K;
+            const int s2 = slot_shift(wc + c + 1, a.n2, a.p);
+            const int u0 = max(4 * b0 - c, 0), u1 = min(4 * (b0 + CB) - c, a.ws);  // window columns [u0, u1)
+            if (u1 <= u0) continue;
+            const int m0 = wrap(u0 + s2, a.ws), n0 = min(u1 - u0, a.ws - m0), n1 = u1 - u0 - n0;
+            if (a.seg == a.K && n1 == 0) {  // whole rows, one after the other
+                copy(out + 4 * c * a.seg, row, nr * a.K);
+            } else {
+                for (int r = 0; r < nr; ++r) {
+                    const float *const src = out + (4 * c + r) * a.seg;
+                    copy(src, row + r * a.K + m0 * a.ws, n0 * a.ws);
+                    if (n1 > 0) copy(src + n0 * a.ws, row + r * a.K, n1 * a.ws);
+                }
             }
         }
     }
@@ -271,11 +291,14 @@ constexpr int strip_of(int nk) { return nk <= 5 ? nk : nk == 6 ? 3 : 2; }
 
 struct SimPlan {
     SimArgs a;
-    int nk, bytes;
+    int nk, qh, bytes;
     bool ok;
 };
-SimPlan sim_plan(const Geom &g, int C, int ncomp, int64_t nb) {
+// qh: query blocks of a wavefront, one above the other (differences: two share
+// the LDS reads of all but two of their block rows)
+SimPlan sim_plan(int qh, const Geom &g, int C, int ncomp, int64_t nb) {
     SimPlan pl{};
+    pl.qh = qh;
     if (g.nsp != 2 || g.p < 1 || g.ws > 33 || g.n1 < g.ws || g.n2 < g.ws || (int64_t)C * ncomp >= 1 << 28 ||
         g.P * g.K * 4 >= kMaxBytes || (int64_t)g.P * C * ncomp * 4 >= kMaxBytes)
         return pl;
@@ -292,7 +315,7 @@ SimPlan sim_plan(const Geom &g, int C, int ncomp, int64_t nb) {
     a.nstrip = (pl.nk + cb - 1) / cb;
     // 4 mod 8 pixels a column, planes 16 mod 32 pixels apart: the 4x4 pixels of
     // four planes fall on 64 banks
-    const int hr = 4 * (kNW + pl.nk - 1);
+    const int hr = 4 * (qh * kNW + pl.nk - 1);
     a.cr = hr + (4 - hr % 8 + 8) % 8;
     const int ncol = 4 * (kNW + cb - 1);
     a.npx = a.cr * ncol;
@@ -303,7 +326,7 @@ SimPlan sim_plan(const Geom &g, int C, int ncomp, int64_t nb) {
     a.region = (16 * a.seg + 1 + 3) / 4 * 4;
     pl.bytes = std::max(16 / ncomp * a.pl, kW * a.region) * 4;
     if (pl.bytes > kLds) return pl;
-    a.tiles_h = (g.n1 + 4 * kNW - 1) / (4 * kNW);
+    a.tiles_h = (g.n1 + 4 * qh * kNW - 1) / (4 * qh * kNW);
     a.tiles_w = (g.n2 + 4 * kNW - 1) / (4 * kNW);
     const int64_t n = (int64_t)a.tiles_h * a.tiles_w * a.nstrip * nb;
     if (n > 1 << 27) return pl;
@@ -317,9 +340,22 @@ SimPlan sim_plan(const Geom &g, int C, int ncomp, int64_t nb) {
     return pl;
 }
 
-template <int NK, bool DIST, bool CPLX>
+// Two query blocks from windows of 19 on, where that leaves two rounds of
+// workgroups or more (us, one block -> two, Distance, 32 components: 4 x 256x254,
+// ws 21 503 -> 415, ws 31 1232 -> 954, 64 components 2180 -> 1620; 2 x 128x126, ws 31,
+// 1280 workgroups of two 171 -> 154, ws 25, 1024, 90 -> 91; 200x120, ws 23, 780, 73 ->
+// 103; at ws 17 whole windows no longer fit: 282 -> 292).
+SimPlan sim_best(bool dist, const Geom &g, int C, int ncomp, int64_t nb) {
+    if (dist && g.ws >= 19) {
+        const SimPlan pl = sim_plan(2, g, C, ncomp, nb);
+        if (pl.ok && pl.a.nitems >= 1200) return pl;
+    }
+    return sim_plan(1, g, C, ncomp, nb);
+}
+
+template <int NK, int QH, bool DIST, bool CPLX>
 hipError_t launch_nk(const SimPlan &pl, hipStream_t s) {
-    auto kern = sim_mx_kernel<NK, strip_of(NK), DIST, CPLX>;
+    auto kern = sim_mx_kernel<NK, strip_of(NK), QH, DIST, CPLX>;
     static const hipError_t e =
         hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     if (e != hipSuccess) return e;
@@ -328,12 +364,13 @@ hipError_t launch_nk(const SimPlan &pl, hipStream_t s) {
 }
 template <bool DIST, bool CPLX>
 hipError_t launch_kind(const SimPlan &pl, hipStream_t s) {
+    constexpr int Q = DIST ? 2 : 1;
     switch (pl.nk) {
-    case 5: return launch_nk<5, DIST, CPLX>(pl, s);
-    case 6: return launch_nk<6, DIST, CPLX>(pl, s);
-    case 7: return launch_nk<7, DIST, CPLX>(pl, s);
-    case 8: return launch_nk<8, DIST, CPLX>(pl, s);
-    case 9: return launch_nk<9, DIST, CPLX>(pl, s);
+    case 5: return launch_nk<5, 1, DIST, CPLX>(pl, s);
+    case 6: return pl.qh == 1 ? launch_nk<6, 1, DIST, CPLX>(pl, s) : launch_nk<6, Q, DIST, CPLX>(pl, s);
+    case 7: return pl.qh == 1 ? launch_nk<7, 1, DIST, CPLX>(pl, s) : launch_nk<7, Q, DIST, CPLX>(pl, s);
+    case 8: return pl.qh == 1 ? launch_nk<8, 1, DIST, CPLX>(pl, s) : launch_nk<8, Q, DIST, CPLX>(pl, s);
+    case 9: return pl.qh == 1 ? launch_nk<9, 1, DIST, CPLX>(pl, s) : launch_nk<9, Q, DIST, CPLX>(pl, s);
     }
     return hipErrorNotSupported;
 }
@@ -345,17 +382,17 @@ hipError_t launch_kind(const SimPlan &pl, hipStream_t s) {
 // against 145) and the sub-row kernel (lines, wider windows).  Measured both ways
 // (us, sub-row kernel -> this one, dot / Distance): 68x60, ws 17, 32 components
 // 119/154 -> 18/36; 200x120, ws 23, 171/213 -> 48/73; 4 x 256x254, ws 17, 434/480 ->
-// 159/282, ws 31 1294/1338 -> 650/1232; with 64 components, where a lane's LDS
-// reads bound the differences, 1500/1674 against 967/2180 (2 x 128x126: 403/520 ->
-// 131/289).
+// 159/282, ws 31 1294/1338 -> 650/954, with 64 components 1500/1674 -> 967/1620;
+// more components cost the differences 21 us each there against 10 (2 x 128x126: 3
+// against 6), so large images of those keep the sub-row kernel.
 bool sim_mx_supported(bool dist, const Geom &g, int C, int ncomp, int64_t nb) {
-    if (g.ws <= 15 || (dist && g.ws > 25 && (int64_t)C * ncomp > 32 && g.P * nb > 100000)) return false;
-    return sim_plan(g, C, ncomp, nb).ok;
+    if (g.ws <= 15 || (dist && g.ws > 25 && (int64_t)C * ncomp > 64 && g.P * nb > 100000)) return false;
+    return sim_best(dist, g, C, ncomp, nb).ok;
 }
 
 hipError_t launch_sim_mx(bool dist, int ncomp, const Geom &g, int C, int64_t nb, float scale, const float *x,
                          const float *y, float *nz, hipStream_t s) {
-    SimPlan pl = sim_plan(g, C, ncomp, nb);
+    SimPlan pl = sim_best(dist, g, C, ncomp, nb);
     if (!pl.ok) return hipErrorNotSupported;
     pl.a.x = x;
     pl.a.y = y;

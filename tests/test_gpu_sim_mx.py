@@ -24,6 +24,9 @@ CASES = [
     ((54, 46), 27, 4, 1, False), ((49, 52), 29, 8, 1, False), ((49, 50), 31, 16, 1, False), ((58, 55), 33, 20, 1, False),
     ((31, 31), 31, 8, 1, False),
     ((30, 27), 17, 1, 2, True), ((45, 41), 17, 17, 1, True), ((36, 41), 21, 8, 1, True), ((52, 46), 23, 3, 1, True), ((52, 55), 31, 10, 1, True),
+    # enough workgroups for two query blocks of a wavefront (Distance)
+    ((101, 90), 19, 4, 9, False), ((60, 67), 23, 5, 9, False), ((61, 57), 27, 4, 10, False),
+    ((58, 60), 33, 2, 10, False), ((90, 101), 21, 2, 9, True),
 ]
 
 
