@@ -18,7 +18,11 @@ from . import _lib as L
 
 
 def stream_ptr(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    # the raw handle: torch.cuda.current_stream builds a Stream object (some 3 us
+    # of a small call's 16) only for its cuda_stream
+    index = torch.device(device).index if device is not None else None
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index))
 
 
 def ptr(t):
