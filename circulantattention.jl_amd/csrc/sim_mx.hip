@@ -76,6 +76,16 @@ __device__ __forceinline__ int wrap(int v, int n) {
     return v - (v >= n ? n : 0);
 }
 
+// Block columns of a wavefront: a window to 17 whole, wider ones in strips whose
+// scores leave registers and LDS for 3 or 4 wavefronts per SIMD.
+constexpr int strip_of(int nk) { return nk <= 5 ? nk : nk == 6 ? 3 : 2; }
+// The queries of a block whose rows are put together at a time: in strips half,
+// since their region of LDS, not the planes, would bound the workgroups of a CU
+// (4 x 256x254, dot, 32 components, ws 21 319 -> 252 us, ws 31 650 -> 575; but whole
+// windows, ws 17, 162 -> 189, and two query blocks, Distance, ws 31, 954 -> 1110,
+// where registers bound them already).
+constexpr int parts_of(int nk, int qh) { return nk >= 6 && qh == 1 ? 2 : 1; }
+
 template <int NK, int CB, int QH, bool DIST, bool CPLX>
 __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
     const int item = (blockIdx.x & 7) * a.per_xcd + (blockIdx.x >> 3);
@@ -242,52 +252,52 @@ __global__ __launch_bounds__(64 * kW, 2) void sim_mx_kernel(SimArgs a) {
             }
         }
     };
+    // (LDS operations of a wavefront are in order)
+    constexpr int NH = parts_of(NK, QH), QR = 16 / NH;
 #pragma unroll
-    for (int b = 0; b < QH; ++b) {  // (LDS operations of a wavefront are in order)
-        {
-            const int s1 = slot_shift(min(rh + 4 * b, a.n1 - 1) + 1, a.n1, a.p);  // (rows past the image: any slots)
-            const int u0 = max(4 * b0 - jc, 0);
-            int col[CB];
+    for (int b = 0; b < QH; ++b) {
+        const int s1 = slot_shift(min(rh + 4 * b, a.n1 - 1) + 1, a.n1, a.p);  // (rows past the image: any slots)
+        const int uj = max(4 * b0 - jc, 0);
+        int col[CB];
 #pragma unroll
-            for (int bc = 0; bc < CB; ++bc) {
-                const int u2 = 4 * (b0 + bc) + g - jc;
-                col[bc] = u2 >= 0 && u2 <= 2 * a.p ? j * a.seg + (u2 - u0) * a.ws : 1 << 24;
-            }
-            const int dump = 16 * a.seg;
-#pragma unroll
-            for (int br = 0; br < NK; ++br)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int u1 = 4 * br + r - jr;
-                    const int m1 = u1 >= 0 && u1 <= 2 * a.p ? wrap(u1 + s1, a.ws) : 1 << 24;
-#pragma unroll
-                    for (int bc = 0; bc < CB; ++bc) out[min(col[bc] + m1, dump)] = acc[b][bc * NK + br][r] * sc;
-                }
+        for (int bc = 0; bc < CB; ++bc) {
+            const int u2 = 4 * (b0 + bc) + g - jc;
+            col[bc] = u2 >= 0 && u2 <= 2 * a.p ? j % QR * a.seg + (u2 - uj) * a.ws : 1 << 24;
         }
+        const int dump = QR * a.seg;
         const int nr = min(4, a.n1 - hw - 4 * b);  // rows of the image
-        for (int c = 0; c < 4; ++c) {
-            if (wc + c >= a.n2 || nr <= 0) break;
-            float *const row = nz + (int64_t)(hw + 4 * b + a.n1 * (wc + c)) * a.K;
-            const int s2 = slot_shift(wc + c + 1, a.n2, a.p);
-            const int u0 = max(4 * b0 - c, 0), u1 = min(4 * (b0 + CB) - c, a.ws);  // window columns [u0, u1)
-            if (u1 <= u0) continue;
-            const int m0 = wrap(u0 + s2, a.ws), n0 = min(u1 - u0, a.ws - m0), n1 = u1 - u0 - n0;
-            if (a.seg == a.K && n1 == 0) {  // whole rows, one after the other
-                copy(out + 4 * c * a.seg, row, nr * a.K);
-            } else {
-                for (int r = 0; r < nr; ++r) {
-                    const float *const src = out + (4 * c + r) * a.seg;
-                    copy(src, row + r * a.K + m0 * a.ws, n0 * a.ws);
-                    if (n1 > 0) copy(src + n0 * a.ws, row + r * a.K, n1 * a.ws);
+        for (int h = 0; h < NH; ++h) {
+            if (j / QR == h) {
+#pragma unroll
+                for (int br = 0; br < NK; ++br)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int u1 = 4 * br + r - jr;
+                        const int m1 = u1 >= 0 && u1 <= 2 * a.p ? wrap(u1 + s1, a.ws) : 1 << 24;
+#pragma unroll
+                        for (int bc = 0; bc < CB; ++bc) out[min(col[bc] + m1, dump)] = acc[b][bc * NK + br][r] * sc;
+                    }
+            }
+            for (int c = QR / 4 * h; c < QR / 4 * (h + 1); ++c) {
+                if (wc + c >= a.n2 || nr <= 0) break;
+                float *const row = nz + (int64_t)(hw + 4 * b + a.n1 * (wc + c)) * a.K;
+                const int s2 = slot_shift(wc + c + 1, a.n2, a.p);
+                const int u0 = max(4 * b0 - c, 0), u1 = min(4 * (b0 + CB) - c, a.ws);  // window columns [u0, u1)
+                if (u1 <= u0) continue;
+                const int m0 = wrap(u0 + s2, a.ws), n0 = min(u1 - u0, a.ws - m0), n1 = u1 - u0 - n0;
+                const float *const from = out + 4 * (c % (QR / 4)) * a.seg;
+                if (a.seg == a.K && n1 == 0) {  // whole rows, one after the other
+                    copy(from, row, nr * a.K);
+                } else {
+                    for (int r = 0; r < nr; ++r) {
+                        copy(from + r * a.seg, row + r * a.K + m0 * a.ws, n0 * a.ws);
+                        if (n1 > 0) copy(from + r * a.seg + n0 * a.ws, row + r * a.K, n1 * a.ws);
+                    }
                 }
             }
         }
     }
 }
-
-// Block columns of a wavefront: a window to 17 whole, wider ones in strips whose
-// scores leave registers and LDS for 3 or 4 wavefronts per SIMD.
-constexpr int strip_of(int nk) { return nk <= 5 ? nk : nk == 6 ? 3 : 2; }
 
 struct SimPlan {
     SimArgs a;
@@ -323,7 +333,7 @@ SimPlan sim_plan(int qh, const Geom &g, int C, int ncomp, int64_t nb) {
     // (halos that wrap once at most)
     if (g.n1 < a.cr - g.p || g.n2 < 4 * (kNW - 1 + a.nstrip * cb) - g.p) return pl;
     a.seg = cb == pl.nk ? a.K : std::min(4 * cb, g.ws) * g.ws;
-    a.region = (16 * a.seg + 1 + 3) / 4 * 4;
+    a.region = (16 / parts_of(pl.nk, qh) * a.seg + 1 + 3) / 4 * 4;
     pl.bytes = std::max(16 / ncomp * a.pl, kW * a.region) * 4;
     if (pl.bytes > kLds) return pl;
     a.tiles_h = (g.n1 + 4 * qh * kNW - 1) / (4 * qh * kNW);
@@ -341,7 +351,7 @@ SimPlan sim_plan(int qh, const Geom &g, int C, int ncomp, int64_t nb) {
 }
 
 // Two query blocks from windows of 19 on, where that leaves two rounds of
-// workgroups or more (us, one block -> two, Distance, 32 components: 4 x 256x254,
+// workgroups or more (us, one block, rows put together whole, -> two, Distance, 32 components: 4 x 256x254,
 // ws 21 503 -> 415, ws 31 1232 -> 954, 64 components 2180 -> 1620; 2 x 128x126, ws 31,
 // 1280 workgroups of two 171 -> 154, ws 25, 1024, 90 -> 91; 200x120, ws 23, 780, 73 ->
 // 103; at ws 17 whole windows no longer fit: 282 -> 292).
@@ -382,7 +392,7 @@ hipError_t launch_kind(const SimPlan &pl, hipStream_t s) {
 // against 145) and the sub-row kernel (lines, wider windows).  Measured both ways
 // (us, sub-row kernel -> this one, dot / Distance): 68x60, ws 17, 32 components
 // 119/154 -> 18/36; 200x120, ws 23, 171/213 -> 48/73; 4 x 256x254, ws 17, 434/480 ->
-// 159/282, ws 31 1294/1338 -> 650/954, with 64 components 1500/1674 -> 967/1620;
+// 159/282, ws 31 1294/1338 -> 575/954, with 64 components 1500/1674 -> 845/1620;
 // more components cost the differences 21 us each there against 10 (2 x 128x126: 3
 // against 6), so large images of those keep the sub-row kernel.
 bool sim_mx_supported(bool dist, const Geom &g, int C, int ncomp, int64_t nb) {
