@@ -191,7 +191,13 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
         if (mode == MODE_FWD) e = launch_f2h2_fwd(pr.g.p, cplx, dist, a, cus, s);
         if (mode == MODE_BWDQ) e = launch_f2h2_bwdq(pr.g.p, cplx, dist, a, cus, s);
         if (mode == MODE_BWDKV) e = launch_f2h2_bwdkv(pr.g.p, cplx, dist, a, cus, s);
-        return e;  // (windows past 11: launch_stream)
+        if (e != hipErrorNotSupported) return e;
+        // Window 15: the Float32 tiles below on images of few pixels, where the
+        // streamed kernels (launch_stream) leave CUs idle (us, forward / backward,
+        // Float32 -> streamed, complex: 128x127 13/36 -> 28/70, 3 units 35/98 ->
+        // 48/124, 256x254 47/131 -> 47/122, 4 units 173/488 -> 144/401; real: 3 x 31x508
+        // 40/105 -> 39/103, 4 units of 256x254 219/565 -> 116/360).
+        if (pr.g.P * pr.nunits > (cplx ? 60000 : 45000)) return hipErrorNotSupported;
     }
     switch (mode) {
     case MODE_FWD: return launch_f2d_fwd(pr.g.p, nt, cplx, dist, a, cus, s);
@@ -219,6 +225,15 @@ hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) 
     const int nt = (ncr + 15) / 16;
     static constexpr int kMinFwd[4] = {400, 49, 25, 15}, kMinBwd[4] = {49, 31, 25, 15};
     if (pr.g.K < (mode == MODE_FWD ? kMinFwd : kMinBwd)[nt - 1]) return hipErrorNotSupported;
+    // Complex components of images that fill the Float32 kernels' grid once but
+    // these kernels' (larger tiles, half the loads' width) barely: us, forward /
+    // backward, Float32 -> these, at 128x127 8 channels, ws 9 -/33 -> -/41, ws 13 -/37 ->
+    // -/45, 16 channels, ws 13 23/62 -> 27/65; 64x63 31 -> 28, 36 -> 39, 23/61 -> 21/51;
+    // 181x180 62 -> 53, 72 -> 59, 44/128 -> 37/90.
+    const int64_t px = pr.g.P * pr.nunits;
+    if (pr.ncomp == 2 && pr.g.nsp == 2 && pr.g.ws <= 13 && (nt == 1 || (nt == 2 && pr.g.ws > 11)) && px > 8000 &&
+        px <= 20000)
+        return hipErrorNotSupported;
     fst::Args a{};
     a.q = pr.q; a.k = pr.k; a.v = pr.v; a.y = pr.y; a.dy = pr.dy; a.lse = pr.lse;
     a.yout = pr.yout; a.lse_out = pr.lse_out; a.dq = pr.dq; a.dk = pr.dk; a.dv = pr.dv;

@@ -39,6 +39,7 @@ CASES = [
     ((300,), 31, 17, 1, 1, 0, False),
     ((150, 130), 9, 32, 2, 2, 0, False),    # workgroups of 8 wavefronts
     ((272, 260), 9, 16, 2, 1, 1, False),    # of 16
+    ((230, 220), 15, 32, 1, 1, 0, False),   # window 15: images past those of the Float32 tiles
 ]
 
 
