@@ -15,9 +15,8 @@
 // What bounds it: dot products by issue (matrix cores a third of the time, the
 // vector instructions of staging and of the rows' assembly a fifth), differences
 // by LDS: a 16-byte read for 8 vector instructions, or 16 where a wavefront
-// takes two query blocks.  200x120, window 23, 32
-// components: 171 -> 48 us, Distance 213 -> 73 us (51 MB of scores, 10 us at the
-// rate of a large copy).
+// takes two query blocks.  200x120, window 23, 32 components: 171 -> 48 us,
+// Distance 213 -> 73 us (51 MB of scores, 10 us at the rate of a large copy).
 #include <algorithm>
 
 #include "circatt_common.h"
@@ -351,10 +350,11 @@ SimPlan sim_plan(int qh, const Geom &g, int C, int ncomp, int64_t nb) {
 }
 
 // Two query blocks from windows of 19 on, where that leaves two rounds of
-// workgroups or more (us, one block, rows put together whole, -> two, Distance, 32 components: 4 x 256x254,
-// ws 21 503 -> 415, ws 31 1232 -> 954, 64 components 2180 -> 1620; 2 x 128x126, ws 31,
-// 1280 workgroups of two 171 -> 154, ws 25, 1024, 90 -> 91; 200x120, ws 23, 780, 73 ->
-// 103; at ws 17 whole windows no longer fit: 282 -> 292).
+// workgroups or more (us, one block, its rows put together whole, -> two;
+// Distance, 32 components: 4 x 256x254, ws 21 503 -> 415, ws 31 1232 -> 954, with 64
+// components 2180 -> 1620; 2 x 128x126, ws 31, 1280 workgroups of two, 171 -> 154,
+// ws 25, 1024, 90 -> 91 (78 in halves); 200x120, ws 23, 780, 73 -> 103; at ws 17 whole
+// windows no longer fit: 282 -> 292).
 SimPlan sim_best(bool dist, const Geom &g, int C, int ncomp, int64_t nb) {
     if (dist && g.ws >= 19) {
         const SimPlan pl = sim_plan(2, g, C, ncomp, nb);
