@@ -225,7 +225,7 @@ int circatt_similarity_bwd(int kind, int dtype, int nsp, int64_t n1, int64_t n2,
     const bool dist = kind == CIRCATT_DISTANCE;
     const float *xf = static_cast<const float *>(x);
     const float *yf = static_cast<const float *>(y);
-    const bool mx = apply_mx_supported(g, (int)C, ncomp, nb);
+    const bool mx = apply_mx_supported(g, (int)C, ncomp, nb, 2);
     if (dx && dy && (mx || apply_pair_supported(g, (int)C, ncomp, nb))) {
         // both products in one grid
         if (dx == x || dx == y) return fail(CIRCATT_ERR_INVALID, "dx must not alias x or y");

@@ -464,23 +464,23 @@ MxPlan mx_plan(const Geom &g, int C, int ncomp, int64_t nb, int products) {
     const int rb = pl.one ? 16 : 4;
     for (int big = 1; big >= 0; --big) {
         const int nwh = pl.one ? (big ? 8 : 4) : (big ? 4 : 2), nww = pl.one ? 1 : 2;
+        MxShape sh{};
         // (two workgroups a CU, or one: room for three gives smaller chunks, 200x120
         // at ws 23: 61 / 71 us, two 54 / 65, one 68 / 87)
         for (int per = 2; per >= 1; --per) {
-            pl.s = mx_shape(pl.one, ncomp == 2, g.p, pl.nt, nwh, nww, kLds / per);
-            if (pl.s.ok) break;
+            sh = mx_shape(pl.one, ncomp == 2, g.p, pl.nt, nwh, nww, kLds / per);
+            if (sh.ok) break;
         }
-        if (!pl.s.ok) continue;
-        // (halos that wrap once at most)
-        if (g.n1 < pl.s.cr - g.p || (!pl.one && g.n2 < 4 * pl.s.cbc * pl.s.nchunk - g.p)) {
-            pl.s.ok = false;
-            continue;
-        }
-        a.tiles_h = (g.n1 + rb * nwh - 1) / (rb * nwh);
-        a.tiles_w = pl.one ? 1 : (g.n2 + 4 * nww - 1) / (4 * nww);
-        const int64_t n = (int64_t)a.tiles_h * a.tiles_w * a.npass * nb;
-        if (n * products > (1 << 27)) return pl;
+        // (halos that wrap once at most: the smaller tiles' wider chunks may
+        // reach further past a narrow image than the larger tiles' do)
+        if (!sh.ok || g.n1 < sh.cr - g.p || (!pl.one && g.n2 < 4 * sh.cbc * sh.nchunk - g.p)) continue;
+        const int th = (g.n1 + rb * nwh - 1) / (rb * nwh), tw = pl.one ? 1 : (g.n2 + 4 * nww - 1) / (4 * nww);
+        const int64_t n = (int64_t)th * tw * a.npass * nb;
+        if (n * products > (1 << 27)) continue;
+        pl.s = sh;
         pl.big = big;
+        a.tiles_h = th;
+        a.tiles_w = tw;
         a.nitems = (int)n;
         if (!big || n * products >= 512) break;
     }
@@ -551,13 +551,13 @@ hipError_t launch_two(const MxPlan &pl, const MxArgs &f, const MxArgs &t, hipStr
 //  - lines from ws 15 on: 65536, ws 15, 32 components 19/24/52 -> 9/10/18; 8 x
 //    65536, ws 63, 64 components 169/184/363 -> 116/126/275; under that 8
 //    components of 8 x 65536 at ws 7 take 22/23/58 against 29/32/72.
-bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb) {
+bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb, int products) {
     const int64_t px = g.P * nb;
     if (g.nsp == 1 ? g.ws < 15
                    : g.ws < 7 || (g.ws <= 15 ? (int64_t)C * ncomp > 16 || px > (1 << 15)
                                              : g.ws <= 31 && px * g.K > 120000000))
         return false;
-    return mx_plan(g, C, ncomp, nb, 2).ok;
+    return mx_plan(g, C, ncomp, nb, products).ok;
 }
 
 #define CIRCATT_MX_SH(F, NT, CPLX, ...)                                                                      \
@@ -612,3 +612,13 @@ hipError_t launch_apply_mx_pair(bool corr, int ncomp, const Geom &g, int C, int6
 }
 
 }  // namespace circatt
+
+// The tiles that a call's products take (1: of 8 wavefronts, 2: of 4; 0: another
+// kernel's call), without a launch; -1 if the rule above sends the call here and
+// the plan refuses it.  For the host tests; no part of the C ABI.
+extern "C" int circatt_route_apply_mx(int nsp, int n1, int n2, int ws, int C, int ncomp, int64_t nb, int products) {
+    const circatt::Geom g = circatt::make_geom(nsp, n1, n2, ws);
+    if (!circatt::apply_mx_supported(g, C, ncomp, nb, products)) return 0;
+    const circatt::MxPlan pl = circatt::mx_plan(g, C, ncomp, nb, products);
+    return !pl.ok ? -1 : pl.big ? 1 : 2;
+}

@@ -43,8 +43,8 @@ hipError_t launch_apply_pair(bool corr, int ncomp, const Geom &g, int C, int64_t
                              const float *nz, const float *x, const float *y, float *dx,
                              float *dy, hipStream_t s);
 // The products on the Float32 matrix cores (apply_mx.hip): wide windows, lines, and
-// few components and pixels
-bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb);
+// few components and pixels; products: 1 (launch_apply_mx) or 2 (the pair)
+bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb, int products);
 hipError_t launch_apply_mx(bool trans, bool corr, int ncomp, const Geom &g, int C, int64_t nb, float scale,
                            const float *nz, const float *x, const float *z, float *y, hipStream_t s);
 hipError_t launch_apply_mx_pair(bool corr, int ncomp, const Geom &g, int C, int64_t nb, float scale, const float *nz,

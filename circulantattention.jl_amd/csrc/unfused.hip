@@ -588,7 +588,7 @@ static hipError_t launch_apply_t(const Geom &g, int C, int64_t nb, float scale, 
 hipError_t launch_apply(bool trans, bool corr, int ncomp, const Geom &g, int C, int64_t nb,
                         float scale, const float *nz, const float *x, const float *z, float *y,
                         hipStream_t s) {
-    if (apply_mx_supported(g, C, ncomp, nb))
+    if (apply_mx_supported(g, C, ncomp, nb, 1))
         return launch_apply_mx(trans, corr, ncomp, g, C, nb, scale, nz, x, z, y, s);
     if (apply_rb_supported(g, C, ncomp, nb))
         return launch_apply_rb(trans, corr, ncomp, g, C, nb, scale, nz, x, z, y, s);

@@ -28,6 +28,8 @@ CASES = [
     ((40, 23), 7, 16, 2, False), ((23, 22), 9, 3, 1, False), ((16, 13), 13, 8, 1, True), ((30, 27), 15, 16, 1, False),
     ((700,), 15, 32, 2, False), ((129,), 63, 40, 1, False), ((200,), 31, 9, 1, True), ((79,), 63, 16, 1, False),
     ((5000,), 127, 70, 1, False), ((140000,), 15, 8, 2, False),
+    # 256 to 511 tiles of 8 wavefronts, none of 4 (their chunks reach past the image)
+    ((195, 43), 27, 8, 4, False), ((512, 31), 17, 32, 2, False), ((145, 29), 19, 8, 8, True),
 ]
 
 
