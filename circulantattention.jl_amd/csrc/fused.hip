@@ -207,7 +207,7 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
     }
 }
 
-// Streamed split-half kernels (fused_stream_impl.h): any window, up to 64 real
+// Streamed kernels (fused_stream_impl.h): any window, up to 64 real
 // components per head; hipErrorNotSupported otherwise.  Buffer offsets are 32
 // bits, and channels-last components are loaded four at a time.
 hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
@@ -251,7 +251,6 @@ hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) 
     a.p = pr.g.p;
     a.pe = 1;
     while (a.pe < 10 && (1 << (a.pe + 1)) < pr.g.K) ++a.pe;
-    a.fine = pr.g.K < 64;
     const bool one = pr.g.nsp == 1, dist = pr.kind == 1;
     const int nu = (int)pr.nunits, cus = device_cus();
 #define CIRCATT_FST_MODE(M)                                        \

@@ -1,4 +1,4 @@
-// Instantiations of the streamed split-half kernels, forward, up to 48 real
+// Instantiations of the streamed kernels, forward, up to 48 real
 // components per head (fused_stream_impl.h).
 #include "fused_stream_impl.h"
 

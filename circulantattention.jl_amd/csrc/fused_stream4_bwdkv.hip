@@ -1,4 +1,4 @@
-// Instantiations of the streamed split-half kernels, key-centric, up to 64 real
+// Instantiations of the streamed kernels, key-centric, up to 64 real
 // components per head (fused_stream_impl.h).
 #include "fused_stream_impl.h"
 

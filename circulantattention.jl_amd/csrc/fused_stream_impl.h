@@ -1,11 +1,17 @@
-// Streamed split-half kernels: fused circulant attention for windows of any
-// width and heads of up to 64 real components, one- and two-dimensional.
+// Streamed kernels: fused circulant attention for windows of any width and
+// heads of up to 64 real components, one- and two-dimensional.
 //
-// Arithmetic.  As in fused2h_impl.h every Float32 operand x is carried as two
-// halves, x = hi + lo with hi = f16(x), lo = f16(x - hi), and a product a.b is
-// taken as hi.hi + lo.hi + hi.lo on v_mfma_f32_16x16x32_f16 with Float32
-// accumulation: 48 cycles for a 16x16 block over 32 components, where
-// v_mfma_f32_16x16x4f32 takes 256.
+// Arithmetic.  Every Float32 operand x is carried as three bf16 thirds,
+// x = a + b + c with a = bf16(x), b the next 8 bits of x - a, c the rest: the
+// sum is exact, as 8 bits each make Float32's 24 and bf16 has its exponents.  A
+// product is taken as the six partial products down to 2^-16 of it on
+// v_mfma_f32_16x16x32_bf16 with Float32 accumulation; those left out (b.c, c.b,
+// c.c) come to 2^-23 of it at most, 2^-26 as a rule, of either sign.  96 cycles for a 16x16 block
+// over 32 components, where v_mfma_f32_16x16x4f32 takes 256.  Two f16 halves
+// (fused2h_impl.h) take 48, but hold an operand to 2^-25 of the largest one that
+// shares its power-of-two scale: a component a thousandth of its neighbours'
+// size would come out with five digits, one of 10^-8 as 0.  Thirds need no scale
+// and treat every component, pixel and magnitude alike.
 //
 // Decomposition.  fused2h_impl.h keeps an item's whole halo in LDS and unrolls
 // the walk over its window, which fits a few (window, components) pairs.  Here
@@ -22,35 +28,44 @@
 // issued into registers before the current chunk's walk.
 //
 // LDS layout.  A slot holds a pixel of both staged tensors,
-// [t0: 64 NT bytes | t1: 64 NT bytes | 32 bytes of pad], each tensor its
-// 32-component groups as [32 hi | 32 lo] halves and a last odd group of 16 as
-// [16 hi | 16 lo].  gfx950 serves a ds_read_b128 in groups of 16 lanes that
+// [t0: 96 NT bytes | t1: 96 NT bytes | 32 bytes of pad], each tensor its
+// 32-component groups as [32 a | 32 b | 32 c] thirds and a last odd group of 16 as
+// [16 a | 16 b | 16 c].  gfx950 serves a ds_read_b128 in groups of 16 lanes that
 // are not consecutive, {0-3, 12-15, 20-27}, {4-11, 16-19, 28-31} and the same
 // plus 32, and ds_read_b64_tr_b16 in two groups of 32 (measured: pairs of
 // lanes on one bank, all others on one address).  With a slot stride of
-// 8 NT + 2 units of 16 bytes and CR = 4 mod 8 slots per column every row read
-// and every transposing read of a block is free of bank conflicts under those
-// groups.
+// 12 NT + 2 units of 16 bytes (2 mod 4) and CR = 4 mod 8 slots per column every row
+// read and every transposing read of a block falls on distinct banks under those
+// groups (tests/test_stream_model.py).
 //
-// What bounds it.  The walk's issue of matrix-core and vector instructions,
-// which add up on a SIMD (a 16x16 block of 32 components: 6 MFMA at 16 cycles
-// in the forward and some 100 cycles of exponentials, splits and sums), is half
-// of the time; the rest is the staging that the walks of one workgroup do not
-// overlap: its loads (the texture path, 14 cycles per 256 bytes), its splits
-// and two barriers per chunk.  Larger tiles stage less per pixel: the shape is
-// the largest that the image fills.  Measured against the Float32 run-time
-// window kernels of fused_impl.h (forward / query- / key-centric pass, us):
-// 512x512, 32 components, Distance, ws 31: 751 / 952 / 1136 -> 300 / 410 / 580;
-// 131x101, 48 components, 2 heads, B = 2, ws 9: 179 / 262 / 314 -> 33 / 38 / 45;
-// 128x96, 64 components, B = 2, ws 15, forward: 102 -> 40; a line of 30011, 64
-// components, B = 4, ws 31: 135 / 354 / 490 -> 38 / 48 / 56; 150x170, 8
-// components, B = 4, ws 9: 51 / 58 / 74 -> 32 / 37 / 46.
+// What bounds it.  On large images the issue of vector and matrix-core
+// instructions, which add up on a SIMD: 512x512, 32 components, Distance, ws 31,
+// forward 0.59 of the time vector and 0.31 matrix-core, query-centric 0.54 and 0.35,
+// key-centric 0.46 and 0.31 and the rest for registers that spill (25 to 80 in the
+// key-centric kernels of 16 wavefronts or 48 and more components with Distance, up
+// to 29 in the query-centric ones of 16; the forward has none).  Images of one round
+// of workgroups are bound by one workgroup's own chain of staging, barriers and
+// walk (0.36 and 0.2 at 2 x 131x101).  Larger tiles stage less per pixel: see the
+// rule at dispatch.  Against the Float32 run-time-window kernels of fused_impl.h
+// (forward / query- / key-centric pass, us): 512x512 as above 720 / 907 / 1115 ->
+// 385 / 495 / 766; 131x101, 48 components, 2 heads, B = 2, ws 9: 179 / 262 / 315 ->
+// 35 / 41 / 51; 128x96, 64 components, B = 2, ws 15: 102 / 127 / 145 -> 47 / 56 / 69; a
+// line of 30011, 64 components, B = 4, ws 31: 124 / 357 / 493 -> 39 / 48 / 56; 150x170, 8
+// components, B = 4, ws 9: 49 / 55 / 70 -> 27 / 31 / 49.  (Halves took 300 / 400 / 567 in the
+// first, 33 / 38 / 46 in the second.)
 //
-// Range.  Staged tensors carry one power-of-two shift for the item so far (the
-// accumulators follow its changes), register operands one for the wavefront, as the f16 halves would lose Float32's range.  Values
-// that a common shift cannot carry (infinities, NaN, outliers and masks of
-// extreme magnitude beside ordinary pixels) send the wavefront's pixels to
-// plain_item, which forms them from Float32 products one pixel at a time.
+// Precision.  Relative 2-norm errors against 64 bits on N(0,1) data, y / dq / dk / dv
+// in units of 1e-7, Float32 kernels -> these: 512x512 as above 8.2 / 11.6 / 10.6 / 9.6 ->
+// 5.8 / 8.8 / 7.1 / 6.5; 131x101 2.7 / 3.5 / 3.4 / 3.3 -> 2.2 / 2.7 / 2.6 / 2.5; 8 components,
+// ws 3 0.95 / 1.8 / 1.7 / 1.5 -> 0.84 / 1.5 / 1.5 / 1.2, ws 21 3.2 / 4.6 / 4.3 / 4.2 ->
+// 1.8 / 2.6 / 2.5 / 2.3; smaller at every window and component count measured.
+//
+// Range.  Staged tensors carry a factor 2^24 and the register partner of a dP
+// product a power of two per pixel, so that the thirds of small values stay
+// normal: magnitudes from 2^-126 to 2^100 are carried exactly.  Anything that is
+// not finite on the way (infinities, NaN, masks near the type's lowest value)
+// leaves a result that is not finite; the wavefront's pixels are then formed by
+// plain_item from Float32 products and their own windows alone.
 #pragma once
 #include "fused2h_impl.h"
 
@@ -66,15 +81,11 @@ using f2d::gmax;
 using f2d::gsum;
 using f2d::kLn2;
 using f2d::kLog2e;
-using f2h::cat;
-using f2h::h2;
-using f2h::h4;
-using f2h::h8;
-using f2h::ldtr;
-using f2h::mfmah;
-using f2h::split2;
-using f2h::split4;
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+typedef unsigned u2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 // vectors at any Float32 address
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
@@ -96,32 +107,62 @@ struct Args {
     float scale, c2;        // similarity scale, scale * log2(e)
     int p;                  // half window
     int pe;                 // exponent PE of the backward's probabilities
-    int fine;               // products include lo.lo (small windows, below)
     int nk;                 // LDS blocks per wavefront along a dimension
     int hr, cr;             // staged rows, LDS column stride (slots)
     int cbc, nchunk;        // block columns per chunk, chunks per item (1, 1 in 1D)
     int npx, wt;            // staged pixels per chunk, wave tasks per chunk
     int os;                 // byte offset of the per-slot scalars
     int om;                 // byte offset of the window masks
-    int ox;                 // byte offset of the exchange words
+    int oc;                 // byte offset of the Distance centre
     int tiles_h, tiles_w, nitems, per_xcd;
     FastDiv div_tiles, div_th, div_nh, div_hr;
+    int *route;             // host only: the shape is written here and nothing launched
 };
 
 template <int NT>
-constexpr int slot_bytes() { return 128 * NT + 32; }
-// byte offset in a tensor's part of a slot of the hi halves of components
-// 16 h .. 16 h + 15, and from them to the lo halves
+constexpr int slot_bytes() { return 192 * NT + 32; }
+// byte offset in a tensor's part of a slot of the first thirds of components
+// 16 h .. 16 h + 15, and from them to the next thirds
 template <int NT>
-constexpr int hi_off(int h) { return 128 * (h >> 1) + ((NT & 1) && h == NT - 1 ? 0 : 32 * (h & 1)); }
+constexpr int third_off(int h) { return 192 * (h >> 1) + ((NT & 1) && h == NT - 1 ? 0 : 32 * (h & 1)); }
 template <int NT>
-constexpr int lo_step(int h) { return (NT & 1) && h == NT - 1 ? 32 : 64; }
+constexpr int third_step(int h) { return (NT & 1) && h == NT - 1 ? 32 : 64; }
 
-// exchange words, (item << 9) | value: largest exponents of what the item has
-// staged so far (tensor 0, centred; tensor 1), 255 - the smallest non-zero
-// exponent of either tensor, the largest exponent of tensor 0 before centring
-// (Distance) and of the staged D (key-centric pass)
-enum { XE0 = 0, XE1 = 1, XM0 = 2, XM1 = 3, XR0 = 4, XD = 5, NXW = 8 };
+__device__ __forceinline__ f4 mfmab(u4 a, u4 b, f4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+// the thirds of two values as packed pairs.  The first is rounded (by one packed
+// conversion), so that the rest, and with it what the products leave out, has
+// either sign; the others are cut off, which is exact for the last.
+__device__ __forceinline__ void split3(float x0, float x1, unsigned &a, unsigned &b, unsigned &c) {
+    constexpr unsigned top = 0xffff0000u, sel = 0x07060302u;  // upper halves of two words
+    a = __builtin_bit_cast(unsigned, __builtin_convertvector((f2{x0, x1}), bf2));
+    const float r0 = x0 - __uint_as_float(a << 16), r1 = x1 - __uint_as_float(a & top);
+    b = __builtin_amdgcn_perm(__float_as_uint(r1), __float_as_uint(r0), sel);
+    const float s0 = r0 - __uint_as_float(__float_as_uint(r0) & top), s1 = r1 - __uint_as_float(__float_as_uint(r1) & top);
+    c = __builtin_amdgcn_perm(__float_as_uint(s1), __float_as_uint(s0), sel);
+}
+template <int N>
+__device__ __forceinline__ void split3(const float (&x)[8], u4 &a, u4 &b, u4 &c) {
+    static_assert(N == 8);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        unsigned u, v, w;
+        split3(x[2 * i], x[2 * i + 1], u, v, w);
+        a[i] = u;
+        b[i] = v;
+        c[i] = w;
+    }
+}
+// transposing LDS reads of four components in two blocks
+__device__ __forceinline__ u4 ldtr2(const char *p0, const char *p1) {
+    const u2 x = __builtin_bit_cast(u2, f2h::ldtr(p0)), y = __builtin_bit_cast(u2, f2h::ldtr(p1));
+    return u4{x[0], x[1], y[0], y[1]};
+}
+
+// Powers of two: of the staged tensors, and of dP' and D' beside the register
+// operand's own (below)
+constexpr int kUp = 24, kUpP = 12;
 
 // One pass over a wavefront's register pixels in Float32, the reference's
 // formulas as they stand: lane c holds component c, one pixel and one window
@@ -188,7 +229,7 @@ __device__ __forceinline__ void plain_item(const Args &a, int64_t uoff, int64_t 
                         L = a.lse[soff + op];
                         D = a.dbuf[soff + op];
                     }
-                    const float e = expf(s - L);
+                    const float e = expf(__builtin_elementwise_minimum(s - L, 0.f));
                     const float ds = e * (wsum(x1 * y1) - D);
                     o0 += ds * (DIST ? y0 - x0 : y0);
                     if constexpr (MODE == BWDKV) o1 += e * y1;
@@ -206,8 +247,7 @@ __device__ __forceinline__ void plain_item(const Args &a, int64_t uoff, int64_t 
     }
 }
 
-// largest magnitude, NaN if any value is (v_maximum3_f32), and its biased
-// exponent (255 for infinities and NaN)
+// largest magnitude and its biased exponent
 template <int N>
 __device__ __forceinline__ float maxabs(const float (&x)[N], float m = 0.f) {
 #pragma unroll
@@ -217,11 +257,6 @@ __device__ __forceinline__ float maxabs(const float (&x)[N], float m = 0.f) {
     return m;
 }
 __device__ __forceinline__ unsigned bexp(float m) { return (__float_as_uint(m) >> 23) & 255u; }
-// maximum over the wave, in an SGPR
-__device__ __forceinline__ unsigned wave_max(unsigned u) {
-    return __builtin_amdgcn_readlane(f2h::wave_umax63(u), 63);
-}
-
 // NT: 16-component groups per pixel; T: wave tasks per wavefront and chunk;
 // CL: channels-last signals (planar: real or complex, a run-time choice of
 // scalar strides)
@@ -229,23 +264,15 @@ template <int NT, int NWH, int NWW, int T, int EU, bool DIST, int MODE, bool ONE
 __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
     constexpr int NW = NWH * NWW;
     constexpr int SB = slot_bytes<NT>();
-    constexpr int T1 = 64 * NT;             // tensor 1's part of a slot
+    constexpr int T1 = 96 * NT;             // tensor 1's part of a slot
     constexpr int NG = (NT + 1) / 2;        // 32-component groups (the last may be a 16)
     constexpr bool ODD = NT & 1;
     constexpr int NTP = NT == 1 ? 1 : NT == 2 ? 2 : 4;  // lanes per staged pixel
     constexpr int PXW = 64 / NTP;           // staged pixels per wave task
     constexpr int RB = ONE ? 16 : 4;        // rows of a block
     constexpr bool KV = MODE == BWDKV;
-    // Backward: probabilities are formed as pt = 2^PE p / rho (below), large
-    // enough for their halves, and dS' = 2^-DE pt (dP' - D').  The staged
-    // tensor 1 and its register partner stay under 2^3, so
-    // |dS'| < 2^(PE + 1 - DE) * 2 * 16 NT * 2^6 <= 2^15.
-    constexpr int DSE = NT == 1 ? 3 : NT == 2 ? 2 : 1;  // PE - DE
-    const int PE = a.pe;
-    const float DEf = __builtin_amdgcn_ldexpf(1.f, DSE - PE);
-    constexpr unsigned HI1 = MODE == FWD ? 131u : 129u;
     char *const lds = reinterpret_cast<char *>(circatt_lds2);
-    unsigned *const xw = reinterpret_cast<unsigned *>(lds + a.ox);
+    float *const cen = reinterpret_cast<float *>(lds + a.oc);
     float *const sc0 = reinterpret_cast<float *>(lds + a.os);
     float *const sc1 = sc0 + (ONE ? 1 : 4 * a.cbc) * a.cr;
 
@@ -254,7 +281,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
     const int j = lane & 15, g = lane >> 4;
     const int jr = ONE ? j : j & 3, jc = ONE ? 0 : j >> 2;
 
-    // score rows: element j of a block, halves 8 g .. 8 g + 7 of a 32-half run
+    // score rows: element j of a block, thirds 8 g .. 8 g + 7 of a run of 32
     const char *const pA = lds + (RB * wh + jr + a.cr * jc) * SB + 16 * g;
     // apply rows by transposing reads: lane j of group g addresses components
     // 4 (j & 3) .. + 3 of element 4 g + (j >> 2): row j >> 2 of column g, or
@@ -292,10 +319,6 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
     auto comp_of = [&](int h, int c) { return (h == NT - 1 ? last0 : 16 * h) + c; };
     auto comp_ok = [&](int h, int c) { return h < NT - 1 || (c >= lastlo && c < lasthi); };
     const bool full = a.ncr == 16 * NT;
-    // Products of groups of 32 leave out lo.lo, some 2^-24 of a product: less
-    // than Float32 sums round over a large window, more than they round over
-    // a small one, where it is formed as well
-    const bool fine = a.fine != 0;
     const int pm = a.lay == PLANAR_C ? 2 : 1;  // floats between pixels (planar)
     // float offset of component c0 + c from c0's, c0 even (planar)
     const int p1 = a.lay == PLANAR_C ? 1 : a.P;
@@ -432,15 +455,22 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
     int k = 0;
     int item = item_of(0);
     if (item >= a.nitems) return;
-    if (threadIdx.x < NXW) xw[threadIdx.x] = 0u;
     int unit, h0, w0;
     decode(item, unit, h0, w0);
     load_stage(unit, h0, w0, 0);
-    // Distance: lane 16 h + c holds component (h, c) of k at the tile's first pixel
+    // Distance: lane 16 h + c holds component (h, c) of the item's centre, the
+    // median of k at the tile's first, middle and last pixel (one outlying
+    // pixel, of whose size the expanded differences would be, does not move it)
     const int mh = min(lane >> 4, NT - 1);
     float nmu = 0.f;
-    if constexpr (DIST) nmu = load1(a.k, unit_off(unit), unit_len(unit), h0 + a.n1 * w0, mh, lane & 15);
-    __syncthreads();  // exchange words cleared
+    auto load_centre = [&](int unit, int h0, int w0) {
+        constexpr int TH = RB * NWH, TW = ONE ? 1 : 4 * NWW;
+        const int hm = min(h0 + TH / 2, a.n1 - 1), wm = ONE ? 0 : min(w0 + TW / 2, a.n2 - 1);
+        const int hl = min(h0 + TH - 1, a.n1 - 1), wl = ONE ? 0 : min(w0 + TW - 1, a.n2 - 1);
+        auto at = [&](int h, int w) { return load1(a.k, unit_off(unit), unit_len(unit), h + a.n1 * w, mh, lane & 15); };
+        return __builtin_amdgcn_fmed3f(at(h0, w0), at(hm, wm), at(hl, wl));
+    };
+    if constexpr (DIST) nmu = load_centre(unit, h0, w0);
 
     while (true) {
         const int64_t uoff = unit_off(unit), soff = (int64_t)unit * a.P;
@@ -448,23 +478,32 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
         const int rh = h0 + RB * wh + jr, rw = w0 + (ONE ? 0 : 4 * ww + jc);
         const bool rvalid = rh < a.n1 && rw < a.n2;
         const int rpix = rvalid ? rh + a.n1 * rw : 0;
-        const unsigned key = (unsigned)k << 9;
         const float cmu = nmu;
 
-        // the wavefront's register operands as halves
-        h8 r0h[NG], r0l[NG], r1h[NG], r1l[NG];
-        bool plain = false;
-        unsigned bq = 0u;
-        int sp = 0, sd = 0;
+        // the wavefront's register operands as thirds (the last odd group of 16,
+        // which a lane holds twice over: a, b, and a in the lower and c in the
+        // upper half of the lane groups)
+        u4 r0[NG][3], r1[NG][3];
+        int sd = 0;
         float rlse = 0.f, rowD = 0.f, sq = 0.f, m = 0.f, rrho = 1.f, ninit = 0.f, fsd = 1.f, kb = 0.f;
-        // backward: p = 2^s / 2^lse2 is formed as pt = 2^(s + PE - I)
-        // with lse2 = I + f, I whole: p = 2^-PE rho pt, rho = 2^-f in (1/2, 1].  The
-        // whole number adds no rounding to the scores, pt is large enough for
-        // its halves where p is not, and rho multiplies the row's results
-        // (query-centric pass) or its staged dy and D (key-centric pass).
+        // backward: p = 2^s / 2^lse2 is formed as pt = 2^(s - I + PE) with lse2 = I + f,
+        // I whole: p = 2^-PE rho pt, rho = 2^-f in (1/2, 1].  The whole number adds no
+        // rounding to the scores, PE (some log2 of the window's slots) keeps the
+        // exponents near 0, where their rounding is least, and rho multiplies the
+        // row's results (query-centric pass) or its staged dy and D (key-centric
+        // pass).
         auto row_split = [&](float lse, float &ipart, float &rho) {
             ipart = floorf(lse * kLog2e);
-            rho = __builtin_amdgcn_exp2f(-__builtin_fmaf(lse, kLog2eLo, __builtin_fmaf(lse, kLog2e, -ipart)));
+            // (the rest of a log-sum-exp of 2^23 and more is its rounding alone)
+            const float f = __builtin_fmaf(lse, kLog2eLo, __builtin_fmaf(lse, kLog2e, -ipart));
+            rho = __builtin_amdgcn_exp2f(-__builtin_amdgcn_fmed3f(f, -1.f, 2.f));
+        };
+        auto rsplit = [&](const float (&x)[NG][8], u4 (&r)[NG][3]) {
+#pragma unroll
+            for (int G = 0; G < NG; ++G) {
+                split3<8>(x[G], r[G][0], r[G][1], r[G][2]);
+                if (ODD && G == NG - 1) r[G][2] = g < 2 ? r[G][0] : r[G][2];
+            }
         };
         {
             float x0[NG][8], x1[NG][8], x2[NG][8];
@@ -489,7 +528,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
             }
             // |q - mu|^2 (k in the key-centric pass); forward: reference score m,
             // the query's own pixel as key (always in its window, so l >= 1)
-            float mr0 = 0.f, mr1 = 0.f;
+            float mr1 = 0.f;
 #pragma unroll
             for (int G = 0; G < NG; ++G) {
                 float s2 = 0.f, dot = 0.f;
@@ -498,7 +537,6 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     if constexpr (DIST) s2 += x0[G][c] * x0[G][c];
                     if constexpr (MODE == FWD) dot += DIST ? x1[G][c] * (x0[G][c] - 0.5f * x1[G][c]) : x0[G][c] * x1[G][c];
                 }
-                mr0 = maxabs(x0[G], mr0);
                 if constexpr (MODE != FWD) mr1 = maxabs(x1[G], mr1);
                 const bool twice = ODD && G == NG - 1 && g >= 2;
                 sq += twice ? 0.f : s2;
@@ -506,15 +544,13 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
             }
             if constexpr (DIST) sq = gsum(sq);
             if constexpr (MODE == FWD) m = gsum(m) * a.c2;
-            // q' = q c2 2^sp with one shift for the wavefront (0 for magnitudes in
-            // [2^-2, 2^5)); a non-finite register operand goes the plain way
-            bq = wave_max(bexp(mr0 * a.c2));
-            plain |= bq == 255u;
-            sp = bq == 0u ? 0 : max(-100, min(100, f2h::shift_of(bq)));
-            auto rsplit = [&](const float (&x)[8], float sc, h8 &hi, h8 &lo) { f2h::reg_split(x, sc, hi, lo); };
+            // q' = q c2 2^-24
+            const float c2s = __builtin_amdgcn_ldexpf(a.c2, -kUp);
 #pragma unroll
-            for (int G = 0; G < NG; ++G) rsplit(x0[G], __builtin_amdgcn_ldexpf(a.c2, sp), r0h[G], r0l[G]);
-            // sd: shift of the register dy (per pixel) or v (one for the wavefront)
+            for (int G = 0; G < NG; ++G)
+#pragma unroll
+                for (int c = 0; c < 8; ++c) x0[G][c] *= c2s;
+            rsplit(x0, r0);
             if constexpr (MODE == BWDQ) {
                 float dd = 0.f;
 #pragma unroll
@@ -525,203 +561,102 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     dd += ODD && G == NG - 1 && g >= 2 ? 0.f : d;  // (held twice)
                 }
                 rowD = gsum(dd);
-                const unsigned b = bexp(gmax(mr1));
-                plain |= __builtin_amdgcn_ballot_w64(bexp(mr1) == 255u || !(fabsf(rowD) < INFINITY) || !(fabsf(rlse) < INFINITY)) != 0;
-                sd = b == 0u ? 0 : max(-100, min(100, 129 - (int)b));
-#pragma unroll
-                for (int G = 0; G < NG; ++G) rsplit(x1[G], __builtin_amdgcn_ldexpf(1.f, sd), r1h[G], r1l[G]);
             }
-            if constexpr (KV) {
-                const unsigned b = wave_max(bexp(mr1));
-                plain |= b == 255u;
-                sd = b == 0u ? 0 : max(-100, min(100, 129 - (int)b));
+            // sd: the power of two that brings the pixel's dy (v) into [4, 8)
+            if constexpr (MODE != FWD) {
+                sd = max(-126, min(114, 129 - (int)bexp(gmax(mr1))));
 #pragma unroll
-                for (int G = 0; G < NG; ++G) rsplit(x1[G], __builtin_amdgcn_ldexpf(1.f, sd), r1h[G], r1l[G]);
+                for (int G = 0; G < NG; ++G)
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) x1[G][c] = __builtin_amdgcn_ldexpf(x1[G][c], sd + kUpP - kUp);
+                rsplit(x1, r1);
             }
             if constexpr (MODE == BWDQ) {
                 float I;
                 row_split(rlse, I, rrho);
-                ninit = PE - I - (DIST ? 0.5f * a.c2 * sq : 0.f);
+                ninit = a.pe - I - (DIST ? 0.5f * a.c2 * sq : 0.f);
             }
-            fsd = KV ? __builtin_amdgcn_ldexpf(1.f, sd) : 1.f;
+            fsd = KV ? __builtin_amdgcn_ldexpf(1.f, sd + kUpP) : 1.f;
             kb = KV && DIST ? -0.5f * a.c2 * sq : 0.f;
         }
-        f4 acc0[NT], acc1[NT];
+        // (one component group: the smaller partial products in a sum of their own,
+        // a second chain and fewer roundings of the large one)
+        constexpr int NA = NT == 1 && !KV ? 2 : 1;
+        f4 acc0[NA][NT], acc1[NA][NT];
 #pragma unroll
-        for (int h = 0; h < NT; ++h) acc0[h] = acc1[h] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int h = 0; h < NT; ++h) acc0[i][h] = acc1[i][h] = f4{0.f, 0.f, 0.f, 0.f};
         float lsum = 0.f, corr = 0.f;
-        int s0 = 0, s1 = 0;
         int xunit = unit, xh0 = h0, xw0 = w0;
         const int nitem = item_of(k + 1);
         const bool has_next = nitem < a.nitems;
 
         for (int ch = 0; ch < a.nchunk; ++ch) {
-            // largest and smallest exponents of what this chunk stages.  The
-            // ballots settle the ordinary case; a wave whose values lie
-            // outside it reduces them
-            bool skew = false;
+            if constexpr (DIST)
+                if (ch == 0 && wv == 0) cen[lane] = cmu;
+            __syncthreads();  // the previous chunk's LDS reads are done; the centre is in
+            // centre, scale, split and store
 #pragma unroll
             for (int i = 0; i < T; ++i) {
                 const int wt = wv + NW * i;
                 if (wt >= a.wt) continue;
                 const bool t1 = wt & 1;
-                unsigned eraw = 0u;
                 FST_FENCE();
+                float up = __builtin_amdgcn_ldexpf(1.f, kUp), sv = 0.f;
                 if constexpr (DIST) {
                     if (!t1) {
-                        eraw = bexp(maxabs(pv[i]));
+                        float q2 = 0.f;
 #pragma unroll
-                        for (int c = 0; c < 16; ++c) pv[i][c] -= __shfl(cmu, 16 * th + c);
-                        if (!full) {
+                        for (int c = 0; c < 16; c += 4) {
+                            const f4 mu = *reinterpret_cast<const f4 *>(cen + 16 * th + c);
 #pragma unroll
-                            for (int c = 0; c < 16; ++c) pv[i][c] = comp_ok(th, c) ? pv[i][c] : 0.f;
+                            for (int e = 0; e < 4; ++e) {
+                                float &x = pv[i][c + e];
+                                x -= mu[e];
+                                if (!full) x = comp_ok(th, c + e) ? x : 0.f;
+                                q2 += x * x;
+                            }
                         }
-                    }
-                }
-                if constexpr (KV) {
-                    bool bad = !(fabsf(pl[i]) < INFINITY);
-                    if (t1) {
-                        float I, rho;
-                        row_split(pl[i], I, rho);
-                        bad |= !(fabsf(pd[i]) < INFINITY);
-                        pd[i] *= rho;
-                        const unsigned ed = wave_max(bexp(pd[i]));
-                        if (lane == 0)
-                            __hip_atomic_fetch_max(xw + XD, key | ed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-#pragma unroll
-                        for (int c = 0; c < 16; ++c) pv[i][c] *= rho;
-                    }
-                    skew |= __builtin_amdgcn_ballot_w64(bad) != 0;
-                }
-                const unsigned e = bexp(maxabs(pv[i]));
-                if constexpr (!DIST) eraw = e;
-                if (t1) eraw = e;
-                const unsigned top = t1 ? HI1 : 131u;
-                const bool odd = __builtin_amdgcn_ballot_w64(e > top || eraw > 138u || (eraw != 0u && eraw < 122u)) != 0 ||
-                                 __builtin_amdgcn_ballot_w64(e >= 125u) == 0;
-                unsigned em = 128u, el = 0u, er = 0u;
-                if (odd) {
-                    em = wave_max(e);
-                    er = wave_max(eraw);
-                    el = wave_max(eraw == 0u ? 0u : 255u - eraw);
-                }
-                if (lane == 0) {
-                    __hip_atomic_fetch_max(xw + (t1 ? XE1 : XE0), key | em, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (odd) {
-                        __hip_atomic_fetch_max(xw + (t1 ? XM1 : XM0), key | el, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-                        if (DIST && !t1)
-                            __hip_atomic_fetch_max(xw + XR0, key | er, __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-                    }
-                }
-            }
-            if constexpr (KV) {
-                if (skew && lane == 0)
-                    __hip_atomic_fetch_max(xw + XE1, key | 255u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            __syncthreads();  // the previous chunk's LDS reads are done; maxima in
-            auto word = [&](int w) __attribute__((always_inline)) {
-                const unsigned x = __builtin_amdgcn_readfirstlane(xw[w]);
-                return (x & ~511u) == key ? x & 511u : 0u;
-            };
-            const unsigned b0 = word(XE0), b1 = word(XE1);
-            const unsigned l0 = word(XM0), l1 = word(XM1);
-            const unsigned br0 = DIST ? max(b0, word(XR0)) : b0;
-            // spread of the pixels' magnitudes (0: not over 2^9), in powers of two
-            const int d0 = l0 ? (int)(br0 + l0) - 255 : 0, d1 = l1 ? (int)(b1 + l1) - 255 : 0;
-            // A small pixel beside large ones keeps 2^(25 + 2) of its spread
-            // with the largest magnitude at [4, 8), and 2^(25 + 12) at
-            // [2^12, 2^13), where spread pixels are taken if the products'
-            // bounds allow it (all but the backward's tensor 1, whose products
-            // become halves again).  What no shift carries goes the plain way:
-            // non-finite values and greater spreads, least where scores are large.
-            plain |= br0 == 255u || b1 == 255u || d0 > 20 || d1 > (MODE == FWD ? 20 : 14);
-            plain |= d0 > 14 && (int)(b0 + bq) - 252 > 12;
-            auto shift = [](unsigned b, unsigned hi, bool wide) {
-                if (b == 0u || (!wide && b >= 125u && b <= hi)) return 0;
-                return max(-100, min(100, (wide ? 139 : 129) - (int)b));
-            };
-            const int n0 = shift(b0, 131u, d0 > 7), n1s = shift(b1, HI1, MODE == FWD && d1 > 7);
-            // the accumulators follow the shifts
-            if (ch > 0 && (n0 != s0 || n1s != s1)) {
-                const int e1 = n1s - s1, e0 = MODE == FWD ? e1 : e1 + n0 - s0;
-#pragma unroll
-                for (int h = 0; h < NT; ++h)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        acc0[h][r] = __builtin_amdgcn_ldexpf(acc0[h][r], e0);
-                        if constexpr (KV) acc1[h][r] = __builtin_amdgcn_ldexpf(acc1[h][r], e1);
-                    }
-                if constexpr (DIST && MODE != FWD) corr = __builtin_amdgcn_ldexpf(corr, e1);
-            }
-            s0 = n0;
-            s1 = n1s;
-
-            // split and store
-#pragma unroll
-            for (int i = 0; i < T; ++i) {
-                const int wt = wv + NW * i;
-                if (wt >= a.wt) continue;
-                const bool t1 = wt & 1;
-                const int sh = t1 ? s1 : s0;
-                FST_FENCE();
-                float q2 = 0.f;
-                if constexpr (DIST) {
-                    if (!t1) {
-#pragma unroll
-                        for (int c = 0; c < 16; ++c) q2 += pv[i][c] * pv[i][c];
                         if constexpr (NTP == 2) q2 += __shfl_xor(q2, 32);
                         if constexpr (NTP == 4) {
                             if (NT == 3 && lane >= 48) q2 = 0.f;
                             q2 = gsum(q2);
                         }
+                        sv = -0.5f * a.c2 * q2;
                     }
                 }
-                if (sh != 0) {
-#pragma unroll
-                    for (int c = 0; c < 16; ++c) pv[i][c] = __builtin_amdgcn_ldexpf(pv[i][c], sh);
+                if constexpr (KV) {
+                    float I, rho;
+                    row_split(pl[i], I, rho);
+                    if (t1) {
+                        sv = -pd[i] * rho;
+                        up *= rho;
+                    } else {
+                        sv += a.pe - I;
+                    }
                 }
-                h2 hi[8], lo[8];
+                u4 st[6];
 #pragma unroll
-                for (int c = 0; c < 8; ++c) split2(pv[i][2 * c], pv[i][2 * c + 1], hi[c], lo[c]);
+                for (int c = 0; c < 8; ++c) {
+                    unsigned x, y, z;
+                    split3(pv[i][2 * c] * up, pv[i][2 * c + 1] * up, x, y, z);
+                    st[c >> 2][c & 3] = x;
+                    st[2 + (c >> 2)][c & 3] = y;
+                    st[4 + (c >> 2)][c & 3] = z;
+                }
                 const int slot = srow[i] + a.cr * scol[i];
                 const bool last16 = ODD && th == NT - 1;
-                char *const sp_ = lds + slot * SB + (t1 ? T1 : 0) + 128 * (th >> 1) + (last16 ? 0 : 32 * (th & 1));
-                char *const sl_ = sp_ + (last16 ? 32 : 64);
+                char *const sp_ = lds + slot * SB + (t1 ? T1 : 0) + 192 * (th >> 1) + (last16 ? 0 : 32 * (th & 1));
                 if (sok[i]) {
 #pragma unroll
-                    for (int c = 0; c < 8; c += 4) {
-                        *reinterpret_cast<f4 *>(sp_ + 4 * c) =
-                            f4{__builtin_bit_cast(float, hi[c]), __builtin_bit_cast(float, hi[c + 1]),
-                               __builtin_bit_cast(float, hi[c + 2]), __builtin_bit_cast(float, hi[c + 3])};
-                        *reinterpret_cast<f4 *>(sl_ + 4 * c) =
-                            f4{__builtin_bit_cast(float, lo[c]), __builtin_bit_cast(float, lo[c + 1]),
-                               __builtin_bit_cast(float, lo[c + 2]), __builtin_bit_cast(float, lo[c + 3])};
-                    }
+                    for (int c = 0; c < 6; ++c)
+                        *reinterpret_cast<u4 *>(sp_ + (c >> 1) * (last16 ? 32 : 64) + 16 * (c & 1)) = st[c];
                     if (th == 0) {
-                        const int si = srow[i] + a.cr * scol[i];
-                        if constexpr (KV) {
-                            if (t1) {
-                                sc1[si] = -__builtin_amdgcn_ldexpf(pd[i], s1);
-                            } else {
-                                float I, rho;
-                                row_split(pl[i], I, rho);
-                                sc0[si] = PE - I - (DIST ? 0.5f * a.c2 * q2 : 0.f);
-                            }
-                        } else if constexpr (DIST) {
-                            if (!t1) sc0[si] = -0.5f * a.c2 * q2;
-                        }
+                        if (KV && t1) sc1[slot] = sv;
+                        if ((KV || DIST) && !t1) sc0[slot] = sv;
                     }
                 }
-            }
-            // D sums over windows that reach past the staged pixels: it is held
-            // to the bound that |dP'| has by its operands
-            if constexpr (MODE != FWD) {
-                const int ed = KV ? (int)word(XD) : (int)wave_max(bexp(rowD));
-                const int es = KV ? ed + s1 + sd : (int)wave_max(bexp(__builtin_amdgcn_ldexpf(rowD, sd + s1)));
-                plain |= ed != 0 && es - 126 > 10 + (NT > 2 ? 2 : NT - 1);
             }
             __syncthreads();  // chunk staged
 
@@ -729,46 +664,69 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
             if (lastch && has_next) decode(nitem, xunit, xh0, xw0);
             load_stage(xunit, xh0, xw0, lastch ? 0 : ch + 1);
             if constexpr (DIST)
-                nmu = load1(a.k, unit_off(xunit), unit_len(xunit), xh0 + a.n1 * xw0, mh, lane & 15);
+                nmu = load_centre(xunit, xh0, xw0);
 
-            const int eu = sp + s0;
-            const float nD = MODE == BWDQ ? -__builtin_amdgcn_ldexpf(rowD, sd + s1) : 0.f;
+            const float ptop = (float)(a.pe + 1);
+            const float nD = MODE == BWDQ ? -__builtin_amdgcn_ldexpf(rowD, sd + kUpP) : 0.f;
 
             // score-type product of a block's 16 pixels with the register
-            // pixels over all components
-            auto score = [&](const char *A, const h8 (&rhi)[NG], const h8 (&rlo)[NG], f4 x) __attribute__((always_inline)) {
+            // pixels over all components: the smaller partial products from 0,
+            // then x0 is added and the largest, so that the sum is rounded at
+            // its full size once for x0 and once for every 32 components
+            auto score = [&](const char *A, const u4 (&r)[NG][3], f4 x0) __attribute__((always_inline)) {
+                f4 x = f4{0.f, 0.f, 0.f, 0.f};
+                u4 t[NG];
 #pragma unroll
                 for (int G = 0; G < NG; ++G) {
-                    const h8 hi = *reinterpret_cast<const h8 *>(A + 128 * G);
+                    const char *const B = A + 192 * G;
+                    t[G] = *reinterpret_cast<const u4 *>(B);
                     if (ODD && G == NG - 1) {
-                        x = mfmah(hi, rhi[G], x);
-                        x = mfmah(hi, rlo[G], x);
+                        // runs of 32: [c | a] on (a, c), [a | b] on (b, b) and (a, a)
+                        const u4 ca = *reinterpret_cast<const u4 *>(B + (g < 2 ? 64 : -32));
+                        x = mfmab(ca, r[G][2], x);
+                        x = mfmab(t[G], r[G][1], x);
                     } else {
-                        const h8 lo = *reinterpret_cast<const h8 *>(A + 128 * G + 64);
-                        if (fine) x = mfmah(lo, rlo[G], x);
-                        x = mfmah(lo, rhi[G], x);
-                        x = mfmah(hi, rlo[G], x);
-                        x = mfmah(hi, rhi[G], x);
+                        const u4 c = *reinterpret_cast<const u4 *>(B + 128);
+                        const u4 b = *reinterpret_cast<const u4 *>(B + 64);
+                        x = mfmab(c, r[G][0], x);
+                        x = mfmab(t[G], r[G][2], x);
+                        x = mfmab(b, r[G][1], x);
+                        x = mfmab(b, r[G][0], x);
+                        x = mfmab(t[G], r[G][1], x);
                     }
                 }
+                x = x + x0;
+#pragma unroll
+                for (int G = 0; G < NG; ++G) x = mfmab(t[G], r[G][0], x);
                 return x;
             };
-            auto apply = [&](const char *R0, const char *R1, h8 ph, h8 pl_, f4 (&acc)[NT]) __attribute__((always_inline)) {
+            // sums of a block pair's pixels, weighted
+            auto apply = [&](const char *R0, const char *R1, const float (&w)[2][4], f4 (&acc)[NA][NT]) __attribute__((always_inline)) {
+                u4 wa, wb, wc;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    unsigned x, y, z;
+                    split3(w[i >> 1][2 * (i & 1)], w[i >> 1][2 * (i & 1) + 1], x, y, z);
+                    wa[i] = x;
+                    wb[i] = y;
+                    wc[i] = z;
+                }
 #pragma unroll
                 for (int h = 0; h < NT; ++h) {
-                    const h8 vh = cat(ldtr(R0 + hi_off<NT>(h)), ldtr(R1 + hi_off<NT>(h)));
-                    const h8 vl = cat(ldtr(R0 + hi_off<NT>(h) + lo_step<NT>(h)),
-                                      ldtr(R1 + hi_off<NT>(h) + lo_step<NT>(h)));
-                    if (NT == 1 || fine) acc[h] = mfmah(vl, pl_, acc[h]);
-                    acc[h] = mfmah(vl, ph, acc[h]);
-                    acc[h] = mfmah(vh, pl_, acc[h]);
-                    acc[h] = mfmah(vh, ph, acc[h]);
+                    FST_FENCE();
+                    const int o = third_off<NT>(h), d = third_step<NT>(h);
+                    const u4 c = ldtr2(R0 + o + 2 * d, R1 + o + 2 * d), b = ldtr2(R0 + o + d, R1 + o + d),
+                             a_ = ldtr2(R0 + o, R1 + o);
+                    f4 &lo = acc[NA - 1][h], &hi = acc[0][h];
+                    lo = mfmab(c, wa, lo);
+                    lo = mfmab(a_, wc, lo);
+                    lo = mfmab(b, wb, lo);
+                    lo = mfmab(b, wa, lo);
+                    lo = mfmab(a_, wb, lo);
+                    hi = mfmab(a_, wa, hi);
                 }
             };
-            // EX: scores unscaled by 2^-eu after the product (and, in the
-            // backward, held to pt <= 2^(PE + 1))
-            auto walk = [&](auto EX, int bc, int cc) __attribute__((always_inline)) {
-                constexpr bool ex = decltype(EX)::value;
+            auto walk = [&](int bc, int cc) __attribute__((always_inline)) {
                 const float cw = ONE ? 0.f : inwin(4 * bc + g - jc);
                 const int co = ONE ? 0 : 4 * cc * a.cr;  // slots before the block column
 #pragma clang loop unroll(disable)
@@ -779,22 +737,21 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     const char *const A0 = pA + o0, *const A1 = pA + o1;
                     const char *const R0 = pR + o0, *const R1 = pR + o1;
                     float p[2][4];
-                    f4 x[2];
                     if constexpr (MODE == FWD) {
+                        // scores less c0 (masked: -inf)
+                        f4 x[2];
+                        auto scores = [&](float c0) __attribute__((always_inline)) {
 #pragma unroll
-                        for (int u = 0; u < 2; ++u) {
-                            const float c = cw - m;
-                            f4 in = pM[MROW * (b + u)] + f4{c, c, c, c};
-                            if constexpr (DIST) in = in + *reinterpret_cast<const f4 *>(pS0 + co + RB * (u && two ? b + 1 : b));
-                            if constexpr (ex) {
-                                const f4 z = score(u ? A1 : A0, r0h, r0l, f4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) x[u][r] = __builtin_amdgcn_ldexpf(z[r], -eu) + in[r];
-                            } else {
-                                x[u] = score(u ? A1 : A0, r0h, r0l, in);
+                            for (int u = 0; u < 2; ++u) {
+                                const float c = cw - c0;
+                                f4 in = pM[MROW * (b + u)] + f4{c, c, c, c};
+                                if constexpr (DIST)
+                                    in = in + *reinterpret_cast<const f4 *>(pS0 + co + RB * (u && two ? b + 1 : b));
+                                FST_FENCE();
+                                x[u] = score(u ? A1 : A0, r0, in);
                             }
-                        }
-                        auto probs = [&]() {
+                        };
+                        auto probs = [&]() __attribute__((always_inline)) {
 #pragma unroll
                             for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -802,30 +759,33 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                             return ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) +
                                    ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
                         };
+                        scores(m);
                         float ps = probs();
                         if (__builtin_amdgcn_ballot_w64(!(ps <= 256.f)) != 0) {
-                            // a score more than 8 above m: m becomes the
-                            // pair's maximum where that is larger
-                            float mx = 0.f;
+                            // a score more than 8 above m: m becomes the pair's
+                            // maximum where that is larger.  The scores are formed
+                            // again without m, of whose rounding they would
+                            // otherwise keep a part if it lay far below them.
+                            scores(0.f);
+                            float mx = m;
 #pragma unroll
                             for (int u = 0; u < 2; ++u)
 #pragma unroll
                                 for (int r = 0; r < 4; ++r) mx = fmaxf(mx, x[u][r]);
                             mx = gmax(mx);
-                            const float f = __builtin_amdgcn_exp2f(-mx);
-                            m += mx;
+                            const float f = __builtin_amdgcn_exp2f(m - mx);
+                            m = mx;
                             lsum *= f;
 #pragma unroll
-                            for (int h = 0; h < NT; ++h) acc0[h] = acc0[h] * f4{f, f, f, f};
+                            for (int i = 0; i < NA; ++i)
+#pragma unroll
+                                for (int h = 0; h < NT; ++h) acc0[i][h] = acc0[i][h] * f4{f, f, f, f};
 #pragma unroll
                             for (int u = 0; u < 2; ++u) x[u] = x[u] - f4{mx, mx, mx, mx};
                             ps = probs();
                         }
                         lsum += ps;
-                        h4 h0_, l0_, h1_, l1_;
-                        split4(p[0], h0_, l0_);
-                        split4(p[1], h1_, l1_);
-                        apply(R0 + T1, R1 + T1, cat(h0_, h1_), cat(l0_, l1_), acc0);
+                        apply(R0 + T1, R1 + T1, p, acc0);
                     } else {
                         float ds[2][4];
 #pragma unroll
@@ -839,42 +799,27 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                                 dp = *reinterpret_cast<const f4 *>(pS1 + co + RB * bb) * f4{fsd, fsd, fsd, fsd};
                             else
                                 dp = f4{nD, nD, nD, nD};
-                            if constexpr (ex) {
-                                const f4 z = score(u ? A1 : A0, r0h, r0l, f4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-                                for (int r = 0; r < 4; ++r)
-                                    x[u][r] = fminf(__builtin_amdgcn_ldexpf(z[r], -eu) + in[r], (float)(PE + 1));
-                            } else {
-                                x[u] = score(u ? A1 : A0, r0h, r0l, in);
-                            }
-                            dp = score((u ? A1 : A0) + T1, r1h, r1l, dp);
+                            FST_FENCE();
+                            const f4 x = score(u ? A1 : A0, r0, in);
+                            dp = score((u ? A1 : A0) + T1, r1, dp);
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
-                                p[u][r] = __builtin_amdgcn_exp2f(x[u][r]);
-                                ds[u][r] = p[u][r] * (dp[r] * DEf);
+                                // (p <= 1: the rounding of very large scores, 2^20 and
+                                // more, would carry some far past it; NaN stays)
+                                p[u][r] = __builtin_amdgcn_exp2f(__builtin_elementwise_minimum(x[r], ptop));
+                                ds[u][r] = p[u][r] * dp[r];
                             }
                             if constexpr (DIST) corr += (ds[u][0] + ds[u][1]) + (ds[u][2] + ds[u][3]);
                         }
-                        h4 h0_, l0_, h1_, l1_;
-                        split4(ds[0], h0_, l0_);
-                        split4(ds[1], h1_, l1_);
-                        apply(R0, R1, cat(h0_, h1_), cat(l0_, l1_), acc0);
-                        if constexpr (KV) {
-                            split4(p[0], h0_, l0_);
-                            split4(p[1], h1_, l1_);
-                            apply(R0 + T1, R1 + T1, cat(h0_, h1_), cat(l0_, l1_), acc1);
-                        }
+                        apply(R0, R1, ds, acc0);
+                        if constexpr (KV) apply(R0 + T1, R1 + T1, p, acc1);
                     }
                 }
             };
-            const bool ex = eu != 0 || (int)(b0 + bq) - 252 > 17;
             for (int cc = 0; cc < (ONE ? 1 : a.cbc); ++cc) {
                 const int bc = ONE ? 0 : ch * a.cbc + cc - ww;
                 if (bc < 0 || bc >= (ONE ? 1 : a.nk)) continue;
-                if (ex)
-                    walk(std::true_type{}, bc, cc);
-                else
-                    walk(std::false_type{}, bc, cc);
+                walk(bc, cc);
             }
         }
 
@@ -890,10 +835,24 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     if (comp_ok(h, 4 * g + r)) o[pm * rpix + coff(c) + coff(r)] = x[r];
             }
         };
-        if (plain) {
+        if constexpr (NA == 2) acc0[0][0] = acc0[0][0] + acc0[1][0];
+        // a result that is not finite: by Float32 products, from the pixels' own
+        // windows (values outside them, and the powers of two, may have made it so)
+        float top = MODE == FWD ? 0.f : fabsf(rlse);
+        bool bad = false;
+#pragma unroll
+        for (int h = 0; h < NT; ++h)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                bad |= !(fabsf(acc0[0][h][r]) < INFINITY);
+                if constexpr (KV) bad |= !(fabsf(acc1[0][h][r]) < INFINITY);
+            }
+        const float l = MODE == FWD ? gsum(lsum) : 1.f;
+        const float cs = DIST && MODE != FWD ? gsum(corr) : 0.f;
+        bad |= !(top < INFINITY) || !(l > 0.f && l < INFINITY) || !(fabsf(m) < INFINITY) || !(fabsf(cs) < INFINITY);
+        if (__builtin_amdgcn_ballot_w64(bad && rvalid) != 0) {
             plain_item<DIST, MODE, ONE>(a, uoff, soff, h0 + RB * wh, w0 + (ONE ? 0 : 4 * ww));
         } else if constexpr (MODE == FWD) {
-            const float l = gsum(lsum);
             float inv = __builtin_amdgcn_rcpf(l);
             inv = __builtin_fmaf(__builtin_fmaf(-l, inv, 1.f), inv, inv);
             if (rvalid) {
@@ -901,26 +860,25 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 for (int h = 0; h < NT; ++h) {
                     float x[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_ldexpf(acc0[h][r] * inv, -s1);
+                    for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_ldexpf(acc0[0][h][r] * inv, -kUp);
                     put4(a.yout, h, x);
                 }
                 if (g == 0) a.lse_out[soff + rpix] = lse_of(m, l, DIST ? 0.5f * sq * a.scale : 0.f);
             }
         } else {
-            const float cs = DIST ? gsum(corr) : 0.f;
 #pragma unroll
             for (int h = 0; h < NT; ++h) {
                 float xk[4], xv[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = __builtin_amdgcn_ldexpf(acc0[h][r], -(sd + s1 + s0) - DSE);
+                    float v = __builtin_amdgcn_ldexpf(acc0[0][h][r], -(sd + kUpP + kUp) - a.pe);
                     if constexpr (DIST) {
                         const float reg = load1(KV ? a.k : a.q, uoff, len, rpix, h, 4 * g + r) -
                                           __shfl(cmu, 16 * h + 4 * g + r);
-                        v -= __builtin_amdgcn_ldexpf(cs, -(sd + s1) - DSE) * reg;
+                        v -= __builtin_amdgcn_ldexpf(cs, -(sd + kUpP) - a.pe) * reg;
                     }
                     xk[r] = v * a.scale * rrho;
-                    if constexpr (KV) xv[r] = __builtin_amdgcn_ldexpf(acc1[h][r], -s1 - PE);
+                    if constexpr (KV) xv[r] = __builtin_amdgcn_ldexpf(acc1[0][h][r], -kUp - a.pe);
                 }
                 if (rvalid) {
                     put4(KV ? a.dk : a.dq, h, xk);
@@ -940,7 +898,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
 
 // Launch shape of a problem; ok = false where it does not fit
 struct Shape {
-    int nk, hr, cr, cbc, nchunk, npx, wt, os, om, ox, bytes;
+    int nk, hr, cr, cbc, nchunk, npx, wt, os, om, oc, bytes;
     bool ok;
 };
 template <int NT, int NWH, int NWW, int T, bool DIST, int MODE, bool ONE>
@@ -962,8 +920,8 @@ inline Shape shape_of(int p, int cap = (int)f2d::kLdsCap) {
         s.wt = 2 * ((s.npx + PXW - 1) / PXW);
         s.os = s.cr * nc * slot_bytes<NT>();
         s.om = s.os + NSC * s.cr * nc * 4;
-        s.ox = s.om + (ONE ? 64 : 4) * 16 * (s.nk + 1);
-        s.bytes = s.ox + NXW * 4;
+        s.oc = s.om + (ONE ? 64 : 4) * 16 * (s.nk + 1);
+        s.bytes = s.oc + (DIST ? 256 : 0);
         if (s.wt <= NW * T && s.bytes <= cap) break;
     }
     s.ok = s.cbc >= 1;
@@ -973,17 +931,21 @@ inline Shape shape_of(int p, int cap = (int)f2d::kLdsCap) {
 template <int NT, int NWH, int NWW, int T, int EU, bool DIST, int MODE, bool ONE, bool CL>
 hipError_t launch_shape(const Args &a0, const Shape &sh, int nunits, int cus, hipStream_t s) {
     constexpr int WH = ONE ? NWH * NWW : NWH, WW = ONE ? 1 : NWW;
-    auto kern = kernel_stream<NT, WH, WW, T, EU, DIST, MODE, ONE, CL>;
-    static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)f2d::kLdsCap);
-    if (attr != hipSuccess) return attr;
     Args a = a0;
     a.nk = sh.nk; a.hr = sh.hr; a.cr = sh.cr; a.cbc = sh.cbc; a.nchunk = sh.nchunk;
-    a.npx = sh.npx; a.wt = sh.wt; a.os = sh.os; a.om = sh.om; a.ox = sh.ox;
+    a.npx = sh.npx; a.wt = sh.wt; a.os = sh.os; a.om = sh.om; a.oc = sh.oc;
     a.tiles_h = (a.n1 + (ONE ? 16 : 4) * WH - 1) / ((ONE ? 16 : 4) * WH);
     a.tiles_w = ONE ? 1 : (a.n2 + 4 * WW - 1) / (4 * WW);
     const int64_t nitems = (int64_t)a.tiles_h * a.tiles_w * nunits;
     if (nitems <= 0 || nitems > (1 << 22)) return hipErrorNotSupported;
+    if (a.route) {
+        *a.route = 10 * NWH + NWW;
+        return hipSuccess;
+    }
+    auto kern = kernel_stream<NT, WH, WW, T, EU, DIST, MODE, ONE, CL>;
+    static const hipError_t attr = hipFuncSetAttribute(
+        reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)f2d::kLdsCap);
+    if (attr != hipSuccess) return attr;
     a.nitems = (int)nitems;
     a.per_xcd = (int)((nitems + 7) / 8);
     a.div_tiles = make_fastdiv((uint32_t)(a.tiles_h * a.tiles_w));
@@ -999,18 +961,28 @@ hipError_t launch_shape(const Args &a0, const Shape &sh, int nunits, int cus, hi
 
 template <int NT, int MODE, bool DIST, bool ONE, bool CL>
 hipError_t dispatch(const Args &a, int nunits, int cus, hipStream_t s) {
+    // tiles of 4 x 2 wavefronts
+    const int64_t tiles = (int64_t)(ONE ? (a.n1 + 127) / 128 : ((a.n1 + 15) / 16) * ((a.n2 + 7) / 8)) * nunits;
+    if constexpr (NT <= 2 && !ONE) {
+        // twice the tile where that saves rounds of workgroups: a round of these
+        // takes some one and a half times as long (one workgroup a CU of either)
+        const Shape b = shape_of<NT, 8, 2, 1, DIST, MODE, ONE>(a.p);
+        const int64_t r8 = (tiles + 2 * cus - 1) / (2 * cus), r4 = (tiles + cus - 1) / cus;
+        if (b.ok && 3 * r8 < 2 * r4 && (MODE != BWDKV || a.p >= 11))
+            return launch_shape<NT, 8, 2, 1, 4, DIST, MODE, ONE, CL>(a, b, nunits, cus, s);
+    }
     const Shape m = shape_of<NT, 4, 2, 3, DIST, MODE, ONE>(a.p);
     // (two workgroups of 4 wavefronts per CU where half of LDS holds a chunk)
     Shape c = shape_of<NT, 2, 2, 3, DIST, MODE, ONE>(a.p, (int)f2d::kLdsCap / 2);
     if (!c.ok) c = shape_of<NT, 2, 2, 3, DIST, MODE, ONE>(a.p);
-    const int64_t px = (int64_t)(ONE ? (a.n1 + 127) / 128 : ((a.n1 + 15) / 16) * ((a.n2 + 7) / 8)) * nunits;
-    if constexpr (NT == 1 || (NT == 2 && MODE != BWDKV)) {
-        const Shape b = shape_of<NT, 8, 2, 1, DIST, MODE, ONE>(a.p);
-        if (!ONE && b.ok && px >= 4LL * cus)
-            return launch_shape<NT, 8, 2, 1, 4, DIST, MODE, ONE, CL>(a, b, nunits, cus, s);
-    }
-    if (m.ok && (px >= cus / 2 || !c.ok)) return launch_shape<NT, 4, 2, 3, 2, DIST, MODE, ONE, CL>(a, m, nunits, cus, s);
+    if (m.ok && (tiles > cus / 2 || !c.ok))
+        return launch_shape<NT, 4, 2, 3, 2, DIST, MODE, ONE, CL>(a, m, nunits, cus, s);
     if (c.ok) return launch_shape<NT, 2, 2, 3, 2, DIST, MODE, ONE, CL>(a, c, nunits, cus, s);
+    if constexpr (NT == 4) {
+        // (the widest windows, whose chunks of the taller tile do not fit LDS)
+        const Shape w = shape_of<NT, 3, 2, 4, DIST, MODE, ONE>(a.p);
+        if (w.ok) return launch_shape<NT, 3, 2, 4, 2, DIST, MODE, ONE, CL>(a, w, nunits, cus, s);
+    }
     return hipErrorNotSupported;
 }
 template <int NT, int MODE>

@@ -64,15 +64,25 @@ int circatt_version(void);
 /*
  * Arithmetic of the fused kernels' matrix products.  The reference computes
  * in Float32 throughout; it has no counterpart of this switch.
- *   CIRCATT_MATH_SPLIT_F16 (default): each Float32 operand is split into two
- *     f16 halves and a product is taken as hi*hi + lo*hi + hi*lo on the f16
- *     matrix cores with Float32 accumulation (relative error near 2^-21 per
- *     operand, the order of Float32 rounding).  Operands are scaled by powers
- *     of two per work item (a 16x16 tile of one head, 8x16 for heads of 32
- *     real components) before the split, so
- *     the halves keep Float32's range: inputs of any magnitude (1e-7 and 1e4
- *     are tested) give Float32-class results.  Where q.k scores are so large
- *     that the halves could overflow, a slower exact-scale walk takes over.
+ *   CIRCATT_MATH_SPLIT_F16 (default): each Float32 operand is split into
+ *     16-bit parts and a product is taken as a sum of partial products on the
+ *     16-bit matrix cores with Float32 accumulation.
+ *     Heads of 16 or 32 real components at the windows that are compiled in
+ *     (2D: 3, 5, 7, 11, and 15 at 16 components; 1D: 15 and 63): two f16 halves,
+ *     hi*hi + lo*hi + hi*lo (relative error near 2^-21 per operand).  Operands
+ *     are scaled by powers of two per work item (a 16x16 tile of one head, 8x16
+ *     for heads of 32 real components, runs of 256 or 128 pixels of a line)
+ *     before the split, so inputs of any magnitude (1e-7 and 1e4 are tested)
+ *     give Float32-class results.  The scale follows the tile's largest value: a
+ *     component far smaller than the others of its tile keeps an absolute error
+ *     of some 2^-27 (at most 2^-23) of that value (four digits at a ratio of 1e-4, none at 1e-8).
+ *     Where q.k scores are so large that the halves could overflow, a slower
+ *     exact-scale walk takes over.
+ *     Other heads of up to 64 real components: three bf16 thirds, which carry a
+ *     Float32 value exactly at every magnitude, and the six partial products
+ *     down to 2^-16 of a product (error 2^-26 of it as a rule): no scale, and
+ *     every component keeps its own precision.
+ *     Calls that neither form takes: Float32 matrix products.
  *   CIRCATT_MATH_F32: Float32 matrix products.
  * Like any attention backward that recomputes the probabilities from the
  * stored log-sum-exp, the fused backward loses precision once scores reach
