@@ -165,85 +165,99 @@ __device__ __forceinline__ u4 ldtr2(const char *p0, const char *p1) {
 constexpr int kUp = 24, kUpP = 12;
 
 // One pass over a wavefront's register pixels in Float32, the reference's
-// formulas as they stand: lane c holds component c, one pixel and one window
-// offset at a time.
-template <bool DIST, int MODE, bool ONE>
+// formulas as they stand: lane j + 16 g holds 4 NT components of pixel j, all
+// lanes one window offset at a time.  Slow, and for values that are not finite
+// alone: with one in every tile 512x512, 32 components, Distance, ws 31 takes 16.5 / 16.6 /
+// 18.3 ms a pass instead of 0.39 / 0.50 / 0.77 (one pixel at a time, a component a
+// lane: 54 / 55 / 103 ms), 131x101, 48 components, 4 units, ws 9 0.41 ms instead of 0.04; the
+// loads, each 16 runs of 4 pixels, bound it.
+template <int NT, bool DIST, int MODE, bool ONE>
 __device__ __forceinline__ void plain_item(const Args &a, int64_t uoff, int64_t soff, int row0, int col0) {
-    const int lane = threadIdx.x & 63;
-    const bool on = lane < a.ncr;
-    auto at = [&](const float *t, int pix) {
-        const int o = a.lay == LAST     ? pix * a.ncrall + lane
-                      : a.lay == PLANAR ? pix + a.P * lane
-                                        : 2 * pix + 2 * a.P * (lane >> 1) + (lane & 1);
-        return on ? t[uoff + o] : 0.f;
+    constexpr int N = 4 * NT;
+    const int j = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const int r = row0 + (ONE ? j : j & 3), c = col0 + (ONE ? 0 : j >> 2);
+    const bool valid = r < a.n1 && c < a.n2;
+    const int pix = valid ? r + a.n1 * c : 0;
+    auto off = [&](int px, int i) {
+        const int k = N * g + i;
+        return a.lay == LAST ? px * a.ncrall + k : a.lay == PLANAR ? px + a.P * k : 2 * px + 2 * a.P * (k >> 1) + (k & 1);
     };
-    auto put = [&](float *t, int pix, float x) {
-        const int o = a.lay == LAST     ? pix * a.ncrall + lane
-                      : a.lay == PLANAR ? pix + a.P * lane
-                                        : 2 * pix + 2 * a.P * (lane >> 1) + (lane & 1);
-        if (on) t[uoff + o] = x;
-    };
-    auto wsum = [](float x) {
+    auto load = [&](const float *t, int px, float (&x)[N]) {
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) x += __shfl_xor(x, d);
-        return x;
+        for (int i = 0; i < N; ++i) x[i] = N * g + i < a.ncr ? t[uoff + off(px, i)] : 0.f;
     };
-    auto score = [&](float x, float y) {
-        const float d = x - y;
-        return DIST ? -0.5f * wsum(d * d) : wsum(x * y);
+    auto put = [&](float *t, const float (&x)[N], float f) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            if (valid && N * g + i < a.ncr) t[uoff + off(pix, i)] = f * x[i];
     };
-    const int p2 = ONE ? 0 : a.p;
-    for (int i = 0; i < 16; ++i) {
-        const int r = row0 + (ONE ? i : i & 3), c = col0 + (ONE ? 0 : i >> 2);
-        if (r >= a.n1 || c >= a.n2) continue;
-        const int pix = r + a.n1 * c;
-        const float x0 = at(MODE == BWDKV ? a.k : a.q, pix);
-        const float xs = DIST ? x0 : x0 * a.scale;  // (scaled first: no overflow the tiled kernels do not have)
-        float x1 = 0.f, D = 0.f, L = 0.f;
-        if constexpr (MODE == BWDQ) {
-            x1 = at(a.dy, pix);
-            D = wsum(x1 * at(a.y, pix));
-            L = a.lse[soff + pix];
-        }
-        if constexpr (MODE == BWDKV) x1 = at(a.v, pix);
-        float m = -INFINITY, l = 0.f, o0 = 0.f, o1 = 0.f;
-        for (int d2 = -p2; d2 <= p2; ++d2)
-            for (int d1 = -a.p; d1 <= a.p; ++d1) {
-                const int op = pmod(r + d1, a.n1) + a.n1 * (ONE ? 0 : pmod(c + d2, a.n2));
-                const float y0 = at(MODE == BWDKV ? a.q : a.k, op);
-                const float y1 = at(MODE == BWDKV ? a.dy : a.v, op);
-                const float s = (DIST ? a.scale : 1.f) * score(xs, y0);
-                if constexpr (MODE == FWD) {
-                    if (s == -INFINITY) continue;
-                    if (!(s <= m)) {
-                        const float f = m == -INFINITY ? 0.f : expf(m - s);
-                        l *= f;
-                        o0 *= f;
-                        m = s;
-                    }
-                    const float e = expf(s - m);
-                    l += e;
-                    o0 += e * y1;
-                } else {
-                    if constexpr (MODE == BWDKV) {
-                        L = a.lse[soff + op];
-                        D = a.dbuf[soff + op];
-                    }
-                    const float e = expf(__builtin_elementwise_minimum(s - L, 0.f));
-                    const float ds = e * (wsum(x1 * y1) - D);
-                    o0 += ds * (DIST ? y0 - x0 : y0);
-                    if constexpr (MODE == BWDKV) o1 += e * y1;
+    auto dot = [&](const float (&x)[N], const float (&y)[N]) {
+        float d = 0.f;
+#pragma unroll
+        for (int i = 0; i < N; ++i) d += x[i] * y[i];
+        return gsum(d);
+    };
+    float x0[N], x1[N], o0[N], o1[N];
+    load(MODE == BWDKV ? a.k : a.q, pix, x0);
+    float m = -INFINITY, l = 0.f, D = 0.f, L = 0.f;
+    if constexpr (MODE == BWDQ) {
+        load(a.y, pix, o0);
+        load(a.dy, pix, x1);
+        D = dot(x1, o0);
+        L = a.lse[soff + pix];
+    }
+    if constexpr (MODE == BWDKV) load(a.v, pix, x1);
+#pragma unroll
+    for (int i = 0; i < N; ++i) o0[i] = o1[i] = 0.f;
+    const int p2 = ONE ? 0 : a.p, first = pmod(r - a.p, a.n1);
+    int c2 = ONE ? 0 : pmod(c - p2, a.n2);
+    for (int d2 = 0; d2 <= 2 * p2; ++d2, c2 = c2 + 1 == a.n2 ? 0 : c2 + 1)
+        for (int d1 = 0, r2 = first; d1 <= 2 * a.p; ++d1, r2 = r2 + 1 == a.n1 ? 0 : r2 + 1) {
+            const int op = r2 + a.n1 * c2;
+            float y0[N], y1[N];
+            load(MODE == BWDKV ? a.q : a.k, op, y0);
+            load(MODE == BWDKV ? a.dy : a.v, op, y1);
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < N; ++i) {
+                const float d = x0[i] - y0[i];
+                // (scaled before the product: no overflow the tiled kernels do not have)
+                s += DIST ? d * d : x0[i] * a.scale * y0[i];
+            }
+            s = gsum(s) * (DIST ? -0.5f * a.scale : 1.f);
+            if constexpr (MODE == FWD) {
+                const bool up = !(s <= m), on = s != -INFINITY;
+                const float f = !up ? 1.f : m == -INFINITY ? 0.f : expf(m - s);
+                if (up) m = s;
+                const float e = on ? expf(s - m) : 0.f;
+                l = l * f + e;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    if (up) o0[i] = f == 0.f ? 0.f : o0[i] * f;
+                    if (on) o0[i] += e * y1[i];
+                }
+            } else {
+                if constexpr (MODE == BWDKV) {
+                    L = a.lse[soff + op];
+                    D = a.dbuf[soff + op];
+                }
+                const float e = expf(__builtin_elementwise_minimum(s - L, 0.f));
+                const float ds = e * (dot(x1, y1) - D);
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    o0[i] += ds * (DIST ? y0[i] - x0[i] : y0[i]);
+                    if constexpr (MODE == BWDKV) o1[i] += e * y1[i];
                 }
             }
-        if constexpr (MODE == FWD) {
-            put(a.yout, pix, o0 / l);
-            if (lane == 0) a.lse_out[soff + pix] = m + logf(l);
-        } else {
-            put(MODE == BWDQ ? a.dq : a.dk, pix, a.scale * o0);
-            if constexpr (MODE == BWDKV) put(a.dv, pix, o1);
-            if constexpr (MODE == BWDQ)
-                if (lane == 0) a.dbuf[soff + pix] = D;
         }
+    if constexpr (MODE == FWD) {
+        put(a.yout, o0, 1.f / l);
+        if (valid && g == 0) a.lse_out[soff + pix] = m + logf(l);
+    } else {
+        put(MODE == BWDQ ? a.dq : a.dk, o0, a.scale);
+        if constexpr (MODE == BWDKV) put(a.dv, o1, 1.f);
+        if constexpr (MODE == BWDQ)
+            if (valid && g == 0) a.dbuf[soff + pix] = D;
     }
 }
 
@@ -453,6 +467,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
         return it < min(a.nitems, (xcd + 1) * a.per_xcd) ? it : a.nitems;
     };
     int k = 0;
+    bool redo = false;
     int item = item_of(0);
     if (item >= a.nitems) return;
     int unit, h0, w0;
@@ -836,8 +851,9 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
             }
         };
         if constexpr (NA == 2) acc0[0][0] = acc0[0][0] + acc0[1][0];
-        // a result that is not finite: by Float32 products, from the pixels' own
-        // windows (values outside them, and the powers of two, may have made it so)
+        // a result that is not finite (values outside the pixel's window, or the
+        // powers of two, may have made it so): NaN marks the wavefront's pixels for
+        // the second pass below
         float top = MODE == FWD ? 0.f : fabsf(rlse);
         bool bad = false;
 #pragma unroll
@@ -850,11 +866,11 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
         const float l = MODE == FWD ? gsum(lsum) : 1.f;
         const float cs = DIST && MODE != FWD ? gsum(corr) : 0.f;
         bad |= !(top < INFINITY) || !(l > 0.f && l < INFINITY) || !(fabsf(m) < INFINITY) || !(fabsf(cs) < INFINITY);
-        if (__builtin_amdgcn_ballot_w64(bad && rvalid) != 0) {
-            plain_item<DIST, MODE, ONE>(a, uoff, soff, h0 + RB * wh, w0 + (ONE ? 0 : 4 * ww));
-        } else if constexpr (MODE == FWD) {
+        const bool again = __builtin_amdgcn_ballot_w64(bad && rvalid) != 0;
+        redo |= again;
+        if constexpr (MODE == FWD) {
             float inv = __builtin_amdgcn_rcpf(l);
-            inv = __builtin_fmaf(__builtin_fmaf(-l, inv, 1.f), inv, inv);
+            inv = again ? NAN : __builtin_fmaf(__builtin_fmaf(-l, inv, 1.f), inv, inv);
             if (rvalid) {
 #pragma unroll
                 for (int h = 0; h < NT; ++h) {
@@ -866,6 +882,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 if (g == 0) a.lse_out[soff + rpix] = lse_of(m, l, DIST ? 0.5f * sq * a.scale : 0.f);
             }
         } else {
+            const float f = again ? NAN : a.scale * rrho;
 #pragma unroll
             for (int h = 0; h < NT; ++h) {
                 float xk[4], xv[4];
@@ -877,7 +894,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                                           __shfl(cmu, 16 * h + 4 * g + r);
                         v -= __builtin_amdgcn_ldexpf(cs, -(sd + kUpP) - a.pe) * reg;
                     }
-                    xk[r] = v * a.scale * rrho;
+                    xk[r] = v * f;
                     if constexpr (KV) xv[r] = __builtin_amdgcn_ldexpf(acc1[0][h][r], -kUp - a.pe);
                 }
                 if (rvalid) {
@@ -893,6 +910,23 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
         unit = xunit;
         h0 = xh0;
         w0 = xw0;
+    }
+    if (!redo) return;
+    // second pass, over the wavefront's marked pixels (here, where the first
+    // pass's registers are free)
+    for (int n = 0; n <= k; ++n) {
+        decode(item_of(n), unit, h0, w0);
+        const int64_t uoff = unit_off(unit);
+        const int rh = h0 + RB * wh + jr, rw = w0 + (ONE ? 0 : 4 * ww + jc);
+        // (component 0, read by the lane that wrote it)
+        bool again = false;
+        if (g == 0 && rh < a.n1 && rw < a.n2) {
+            const int pix = rh + a.n1 * rw;
+            const float x = (MODE == FWD ? a.yout : MODE == BWDQ ? a.dq : a.dk)[uoff + (CL ? pix * a.ncrall : pm * pix)];
+            again = x != x;
+        }
+        if (__builtin_amdgcn_ballot_w64(again) != 0)
+            plain_item<NT, DIST, MODE, ONE>(a, uoff, (int64_t)unit * a.P, h0 + RB * wh, w0 + (ONE ? 0 : 4 * ww));
     }
 }
 

@@ -122,6 +122,30 @@ def test_stream_extreme_pixel(ca, cuda, dims, ws, C, kind, which, value, first):
             assert abs_err(a, b) <= bar
 
 
+@pytest.mark.parametrize("dims,ws,C,kind", [((400, 390), 9, 32, 0), ((60000,), 31, 48, 1)])
+def test_stream_nan_in_several_items(ca, cuda, dims, ws, C, kind):  # noqa: F811
+    """Workgroups of two and more items each, the second pass over some of them:
+    NaN in v at scattered pixels."""
+    sim = ca.DistanceSimilarity() if kind else ca.DotSimilarity()
+    shape = shape_of(dims, C, 1)
+    xs = [seeded(70 + i, shape) for i in range(4)]
+    spots = np.random.default_rng(7).integers(0, shape[2:], (40, len(dims)))
+    t = [dev(x, cuda) for x in xs]
+    dist = np.full(shape[2:], 1 << 20)
+    for at in spots:
+        t[2][(0, slice(None), *map(int, at))] = float("nan")
+        dist = np.minimum(dist, distance_from(shape[2:], at))
+    t = [x.requires_grad_(i < 3) for i, x in enumerate(t)]
+    y, _ = ca.circulant_mh_attention(sim, *t[:3], ws, 1, materialize=False, honor_simfun=True)
+    got = [host(z) for z in (y, *torch.autograd.grad(y, t[:3], t[3]))]
+    ref = [O.attention_fwd(kind, *xs[:3], ws, 1)[0], *O.attention_bwd(kind, *xs, ws, 1)]
+    p = ws // 2
+    for i, (a, b) in enumerate(zip(got, ref)):
+        far = dist > (2 * p if i >= 2 else p)
+        assert rel_err(a[0][:, far], b[0][:, far]) < (1e-5 if i == 0 else 1e-4)
+        assert np.isnan(a[0][:, dist == 0]).all() if i < 2 else True
+
+
 @pytest.mark.parametrize("dims,ws,C", [((60, 50), 9, 48), ((60, 50), 31, 32), ((60, 50), 15, 64), ((2000,), 31, 64)])
 def test_stream_error_rms(ca, cuda, dims, ws, C):  # noqa: F811
     """Relative 2-norm errors against 64 bits.  A row's probabilities carry the
