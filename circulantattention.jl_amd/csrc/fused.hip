@@ -141,17 +141,38 @@ bool fused_supported(FusedMode mode, const FusedProblem &pr) {
     return pl.ok || make_wide_plan(mode, pr).ok;
 }
 
-// Compile-time-window 2D kernels (fused2d_impl.h) for the shapes they cover;
-// hipErrorNotSupported otherwise.
-hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
+// tiles of n x n pixels (runs of n n in one dimension) of all units
+int64_t tiles_of(const FusedProblem &pr, int n) {
+    const int64_t t = pr.g.nsp == 1 ? (pr.g.n1 + n * n - 1) / (n * n)
+                                    : (int64_t)((pr.g.n1 + n - 1) / n) * ((pr.g.n2 + n - 1) / n);
+    return t * pr.nunits;
+}
+
+// Whether the compile-time-window kernels (fused2d_impl.h, fused2h_impl.h) take a
+// shape.
+bool takes_f2d(FusedMode mode, const FusedProblem &pr) {
     const int ncr = pr.dh * pr.ncomp;
+    if (mode == MODE_SIM || pr.nunits > INT32_MAX) return false;
+    const bool split = math_mode() == CIRCATT_MATH_SPLIT_F16;
     // one-dimensional signals: the split-half kernels of the windows they
     // instantiate (no Float32 matrix-core counterpart)
-    const bool one = pr.g.nsp == 1 && math_mode() == CIRCATT_MATH_SPLIT_F16 &&
-                     f2h::supported1(pr.g.p, ncr) && pr.g.P * ncr * 4 < (int64_t)INT32_MAX;
-    if (mode == MODE_SIM || !(one || f2d::supported(pr.g.nsp, pr.g.p, ncr, pr.g.P)) ||
-        pr.nunits > INT32_MAX)
-        return hipErrorNotSupported;
+    if (pr.g.nsp == 1)
+        return split && f2h::supported1(pr.g.p, ncr) && pr.g.P * ncr * 4 < (int64_t)INT32_MAX;
+    if (!f2d::supported(pr.g.nsp, pr.g.p, ncr, pr.g.P)) return false;
+    // Window 15 at 32 real components on at least as many 16x16 tiles as CUs: the
+    // streamed kernels (launch_stream), whose 32x8 tiles then fill the CUs as well.
+    // us, forward / backward, Float32 tiles -> streamed, Dot: 128x127 16/40 -> 27/68,
+    // 192x192 38/101 -> 36/114, 256x254 57/146 -> 39/122, 320x320 87/232 -> 70/217, 4 x
+    // 256x254 217/567 -> 140/442; Distance: 192x192 40/107 -> 45/139, 256x254 60/154 ->
+    // 48/151, 320x320 92/248 -> 87/268, 4 x 256x254 232/605 -> 176/546.  Complex components,
+    // whose planar loads are half as wide, stay: 256x254 46/127 against 46/136, 4 units
+    // 172/490 against 164/488, Distance 188/524 against 199/582.
+    return !(split && ncr == 32 && pr.g.p == 7 && pr.ncomp == 1 && tiles_of(pr, 16) >= device_cus());
+}
+
+hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
+    const int ncr = pr.dh * pr.ncomp;
+    const bool one = pr.g.nsp == 1;
     f2d::Args a{};
     a.q = pr.q; a.k = pr.k; a.v = pr.v; a.y = pr.y; a.dy = pr.dy; a.lse = pr.lse;
     a.yout = pr.yout; a.lse_out = pr.lse_out; a.dq = pr.dq; a.dk = pr.dk; a.dv = pr.dv;
@@ -192,12 +213,6 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
         if (mode == MODE_BWDQ) e = launch_f2h2_bwdq(pr.g.p, cplx, dist, a, cus, s);
         if (mode == MODE_BWDKV) e = launch_f2h2_bwdkv(pr.g.p, cplx, dist, a, cus, s);
         if (e != hipErrorNotSupported) return e;
-        // Window 15: the Float32 tiles below on images of few pixels, where the
-        // streamed kernels (launch_stream) leave CUs idle (us, forward / backward,
-        // Float32 -> streamed, complex: 128x127 13/36 -> 28/70, 3 units 35/98 ->
-        // 48/124, 256x254 47/131 -> 47/122, 4 units 173/488 -> 144/401; real: 3 x 31x508
-        // 40/105 -> 39/103, 4 units of 256x254 219/565 -> 116/360).
-        if (pr.g.P * pr.nunits > (cplx ? 60000 : 45000)) return hipErrorNotSupported;
     }
     switch (mode) {
     case MODE_FWD: return launch_f2d_fwd(pr.g.p, nt, cplx, dist, a, cus, s);
@@ -210,29 +225,27 @@ hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
 // Streamed kernels (fused_stream_impl.h): any window, up to 64 real
 // components per head; hipErrorNotSupported otherwise.  Buffer offsets are 32
 // bits, and channels-last components are loaded four at a time.
-hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
+hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s, int *route = nullptr) {
     const int ncr = pr.dh * pr.ncomp;
     const int64_t all = (int64_t)pr.nheads * ncr;
     if (mode == MODE_SIM || math_mode() != CIRCATT_MATH_SPLIT_F16 || ncr > 64 || pr.nunits > INT32_MAX ||
         pr.g.p < 1 || pr.g.P * (pr.cl ? all : ncr) * 4 >= (int64_t)fst::kMaxBytes || (pr.cl && ncr % 4 != 0))
         return hipErrorNotSupported;
-    // Windows of fewer keys stay on the Float32 products: there the halves'
-    // error (2^-24 to 2^-23 of a product) is the larger (measured against 64
-    // bits on N(0,1) data, errors of y at 8, 16 components: 1.34 x at ws 3,
-    // 1.13 x at ws 9, below 1 x from ws 23; 48, 64: 1.2 x at ws 3, at most 1 x
-    // from ws 5; gradients, whose probabilities this family rounds less, below
-    // 1 x from ws 7 at 8 components).
     const int nt = (ncr + 15) / 16;
-    static constexpr int kMinFwd[4] = {400, 49, 25, 15}, kMinBwd[4] = {49, 31, 25, 15};
-    if (pr.g.K < (mode == MODE_FWD ? kMinFwd : kMinBwd)[nt - 1]) return hipErrorNotSupported;
-    // Complex components of images that fill the Float32 kernels' grid once but
-    // these kernels' (larger tiles, half the loads' width) barely: us, forward /
-    // backward, Float32 -> these, at 128x127 8 channels, ws 9 -/33 -> -/41, ws 13 -/37 ->
-    // -/45, 16 channels, ws 13 23/62 -> 27/65; 64x63 31 -> 28, 36 -> 39, 23/61 -> 21/51;
-    // 181x180 62 -> 53, 72 -> 59, 44/128 -> 37/90.
-    const int64_t px = pr.g.P * pr.nunits;
-    if (pr.ncomp == 2 && pr.g.nsp == 2 && pr.g.ws <= 13 && (nt == 1 || (nt == 2 && pr.g.ws > 11)) && px > 8000 &&
-        px <= 20000)
+    // Any window and component count, with these exceptions: images of at most one
+    // 8x8 tile of the Float32 kernels a CU, at windows whose 4x4 blocks reach furthest
+    // past them (ws 7: 144 slots for 49, ws 11 and 13: 256 for 121 and 169; window 15 is
+    // compiled into the Float32 kernel of 16 components).  us, forward + backward,
+    // Float32 -> these, 128x127, Dot / Distance, 8 components: ws 3 34 -> 30 / 36 -> 34,
+    // ws 5 34 -> 29 / 37 -> 33, ws 7 37 -> 37 / 39 -> 42, ws 9 46 -> 34 / 53 -> 38, ws 11
+    // 52 -> 52 / 56 -> 60, ws 13 53 -> 52 / 59 -> 60, ws 15 52 -> 68 / 67 -> 78, ws 17 87 ->
+    // 62 / 96 -> 74; 4 complex ones: ws 7 35 -> 41 / 39 -> 46, ws 9 49 -> 40 / 54 -> 48,
+    // ws 13 53 -> 57 / 59 -> 63; 24: ws 7 51 -> 52 / 55 -> 60, ws 11 78 -> 67 / 84 -> 80; 12
+    // complex ones: ws 7 50 -> 58 / 55 -> 68, ws 13 87 -> 74 / 93 -> 88.  Two units of
+    // that size: 8 components, ws 7 50 -> 47 / 53 -> 53, ws 13 72 -> 52 / 78 -> 60, ws 15
+    // 70 -> 72 / 91 -> 84; 24, ws 7 72 -> 61 / 79 -> 71.
+    if (pr.g.nsp == 2 && ((nt <= 2 && pr.g.ws == 7) || (nt == 1 && pr.g.ws >= 11 && pr.g.ws <= 15)) &&
+        tiles_of(pr, 8) <= device_cus())
         return hipErrorNotSupported;
     fst::Args a{};
     a.q = pr.q; a.k = pr.k; a.v = pr.v; a.y = pr.y; a.dy = pr.dy; a.lse = pr.lse;
@@ -249,6 +262,7 @@ hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) 
     a.scale = pr.scale;
     a.c2 = pr.scale * kLog2e;
     a.p = pr.g.p;
+    a.route = route;
     a.pe = 1;
     while (a.pe < 10 && (1 << (a.pe + 1)) < pr.g.K) ++a.pe;
     const bool one = pr.g.nsp == 1, dist = pr.kind == 1;
@@ -268,7 +282,7 @@ hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s) 
 
 hipError_t launch_fused(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
     if (mode != MODE_SIM) {
-        hipError_t e = launch_f2d(mode, pr, s);
+        hipError_t e = takes_f2d(mode, pr) ? launch_f2d(mode, pr, s) : hipErrorNotSupported;
         if (e == hipErrorNotSupported) e = launch_stream(mode, pr, s);
         if (e != hipErrorNotSupported) return e;
     }
@@ -289,3 +303,24 @@ hipError_t launch_fused(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
 }
 
 }  // namespace circatt
+
+// The kernel that a fused call takes, without a launch: 1 for the compile-time
+// windows, 10 H + W for the streamed kernels' workgroups of H x W wavefronts, 0 for
+// the general kernels.  For the tests; no part of the C ABI.
+extern "C" int circatt_route_fused(int mode, int kind, int ncomp, int nsp, int n1, int n2, int ws, int dh, int nheads,
+                                   int64_t nunits, int channels_last) {
+    circatt::FusedProblem pr{};
+    pr.g = circatt::make_geom(nsp, n1, n2, ws);
+    pr.kind = kind;
+    pr.ncomp = ncomp;
+    pr.dh = dh;
+    pr.nunits = nunits;
+    pr.nheads = nheads;
+    pr.cl = channels_last;
+    pr.scale = 1.f;
+    const circatt::FusedMode m = mode == 0 ? circatt::MODE_FWD : mode == 1 ? circatt::MODE_BWDQ : circatt::MODE_BWDKV;
+    if (circatt::takes_f2d(m, pr)) return 1;
+    int route = 0;
+    circatt::launch_stream(m, pr, nullptr, &route);
+    return route;
+}

@@ -995,18 +995,34 @@ hipError_t launch_shape(const Args &a0, const Shape &sh, int nunits, int cus, hi
 
 template <int NT, int MODE, bool DIST, bool ONE, bool CL>
 hipError_t dispatch(const Args &a, int nunits, int cus, hipStream_t s) {
-    // tiles of 4 x 2 wavefronts
+    // Tiles of 4 x 2 wavefronts; workgroups of these are one a CU in most cases.
+    // us, forward / query- / key-centric pass, at the crossings:
+    //   tiles    shape                      2 x 2          4 x 2         8 x 2
+    //   96       32 components, ws 9        14/16/19       15/17/21
+    //            64, ws 15                  40/44/54       44/51/63
+    //   144      32, ws 9                   16/19/22       16/17/22
+    //            64, ws 15                  70/79/98       44/52/63
+    //   256      32, ws 17                  31/37/45       25/31/39      34/42/64
+    //   288      32, ws 9                   25/29/34       27/32/39      21/26/41
+    //            32, ws 31, Distance        136/156/185    149/173/204   96/122/180
+    //   512      32, ws 17                  56/66/83       45/55/69      38/48/78
+    //            32, ws 31, Distance        165/187/225    153/178/208   101/136/202
+    //   544      32, ws 17                  69/83/103      64/79/98      67/85/133
+    //   1536     32, ws 17                  155/188/234    126/153/193   102/130/210
+    //            32, ws 31, Distance        471/543/654    450/522/615   283/371/572
+    // (8 x 2 in the key-centric pass spills registers, which narrow windows repay less)
     const int64_t tiles = (int64_t)(ONE ? (a.n1 + 127) / 128 : ((a.n1 + 15) / 16) * ((a.n2 + 7) / 8)) * nunits;
     if constexpr (NT <= 2 && !ONE) {
         // twice the tile where that saves rounds of workgroups: a round of these
-        // takes some one and a half times as long (one workgroup a CU of either)
+        // takes some one and a half times as long
         const Shape b = shape_of<NT, 8, 2, 1, DIST, MODE, ONE>(a.p);
         const int64_t r8 = (tiles + 2 * cus - 1) / (2 * cus), r4 = (tiles + cus - 1) / cus;
         if (b.ok && 3 * r8 < 2 * r4 && (MODE != BWDKV || a.p >= 11))
             return launch_shape<NT, 8, 2, 1, 4, DIST, MODE, ONE, CL>(a, b, nunits, cus, s);
     }
     const Shape m = shape_of<NT, 4, 2, 3, DIST, MODE, ONE>(a.p);
-    // (two workgroups of 4 wavefronts per CU where half of LDS holds a chunk)
+    // half the tile up to half a round, two workgroups a CU where half of LDS
+    // holds a chunk
     Shape c = shape_of<NT, 2, 2, 3, DIST, MODE, ONE>(a.p, (int)f2d::kLdsCap / 2);
     if (!c.ok) c = shape_of<NT, 2, 2, 3, DIST, MODE, ONE>(a.p);
     if (m.ok && (tiles > cus / 2 || !c.ok))

@@ -4,12 +4,16 @@ sizes where they can go wrong.
 Component counts that fill no whole group of 16 (the last group then overlaps
 the one before, or repeats a component), windows between and past those of the
 compile-time-window kernels, images narrower than the window and than a tile,
-odd sizes and every layout.  The bar is the repository's (1e-5 forward, 1e-4 gradients, max-norm
+odd sizes, every layout, and images large enough for each workgroup shape; each
+case names the shape that it is there for, and the library is asked which it
+takes.  The bar is the repository's (1e-5 forward, 1e-4 gradients, max-norm
 relative).  Further tests: channels far smaller than their neighbours, each
 held to its own size; magnitudes from 1e-7 to 1e4; one pixel of one tensor
 extreme or not finite, which must not disturb a pixel whose window it is not in;
 and the error's 2-norm over small and wide windows against a bound derived from
 the roundings."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -23,6 +27,17 @@ pytestmark = pytest.mark.gpu
 
 import oracle as O  # noqa: E402
 from test_gpu_magnitudes import MAGS, _across_magnitudes  # noqa: E402
+
+
+def routes(dims, ws, C, B, nh, kind, cplx, last=False):
+    """Workgroup shapes (10 H + W wavefronts; 0, 1: other kernels) of the forward
+    and the two backward passes."""
+    from circulant_attention import _lib as L
+    n1, n2 = dims if len(dims) == 2 else (dims[0], 1)
+    f = L.lib.circatt_route_fused
+    f.argtypes = [ctypes.c_int] * 9 + [ctypes.c_int64, ctypes.c_int]
+    return tuple(f(m, kind, 2 if cplx else 1, len(dims), n1, n2, ws, C // nh, nh, nh * B, last) for m in range(3))
+
 
 # (spatial, ws, C, B, nheads, kind, complex)
 CASES = [
@@ -41,12 +56,29 @@ CASES = [
     ((300,), 31, 17, 1, 1, 0, False),
     ((31, 26), 3, 24, 1, 1, 0, False), ((100, 90), 7, 5, 2, 1, 1, False),  # the smallest windows
 ]
+# (..., workgroup shapes of the three passes)
+SHAPE_CASES = [
+    ((150, 130), 9, 32, 2, 2, 0, False, (42, 42, 42)), ((20000,), 31, 17, 1, 1, 1, False, (42, 42, 42)),
+    ((200, 190), 9, 32, 1, 1, 0, False, (82, 82, 42)), ((200, 190), 21, 16, 1, 1, 0, False, (82, 82, 42)),
+    ((272, 260), 9, 16, 2, 1, 1, False, (82, 82, 42)), ((200, 190), 17, 8, 1, 1, 0, True, (82, 82, 42)),
+    ((193, 190), 23, 32, 1, 1, 0, False, (82, 82, 82)), ((200, 187), 23, 16, 1, 1, 1, True, (82, 82, 82)),
+    ((256, 250), 15, 32, 1, 1, 0, False, (82, 82, 42)),  # window 15: past the Float32 tiles' one round
+    ((40, 30), 31, 64, 1, 1, 1, False, (32, 32, 32)), ((500,), 63, 64, 1, 1, 0, False, (42, 42, 32)),
+]
 
 
 @pytest.mark.parametrize("case", CASES, ids=lambda c: f"{'x'.join(map(str, c[0]))}-ws{c[1]}-C{c[2]}-B{c[3]}-h{c[4]}-"
                                                      f"{'dist' if c[5] else 'dot'}-{'c32' if c[6] else 'f32'}")
 def test_stream_against_oracle(ca, cuda, case):  # noqa: F811
     dims, ws, C, B, nh, kind, cplx = case
+    assert min(routes(*case)) >= 22
+    _attention_case(ca, cuda, dims, ws, C, B, nh, 700 + C + ws, cplx, kind, materialize=False)
+
+
+@pytest.mark.parametrize("case", SHAPE_CASES, ids=lambda c: f"{'x'.join(map(str, c[0]))}-ws{c[1]}-C{c[2]}-{c[7]}")
+def test_stream_shapes_against_oracle(ca, cuda, case):  # noqa: F811
+    dims, ws, C, B, nh, kind, cplx, shapes = case
+    assert routes(*case[:7]) == shapes
     _attention_case(ca, cuda, dims, ws, C, B, nh, 700 + C + ws, cplx, kind, materialize=False)
 
 
@@ -56,6 +88,7 @@ def test_stream_against_oracle(ca, cuda, case):  # noqa: F811
 @pytest.mark.parametrize("mag", MAGS)
 @pytest.mark.parametrize("kind", [0, 1])
 def test_stream_across_magnitudes(ca, cuda, case, which, mag, kind):  # noqa: F811
+    assert min(routes(*case, kind, False)) >= 22
     _across_magnitudes(ca, cuda, case, which, mag, False, kind, 300)
 
 
@@ -65,6 +98,7 @@ def test_stream_across_magnitudes(ca, cuda, case, which, mag, kind):  # noqa: F8
 def test_stream_channels_last(ca, cuda, dims, ws, C, nh, kind, cplx):  # noqa: F811
     """The layouts carry the same values through the same arithmetic."""
     sim = ca.DistanceSimilarity() if kind else ca.DotSimilarity()
+    assert min(routes(dims, ws, C, 2, nh, kind, cplx, True)) >= (82 if dims[0] == 150 else 22)
     xs = [dev(seeded(40 + i, shape_of(dims, C, 2), cplx), cuda) for i in range(4)]
     out = []
     for last in (False, True):
@@ -101,6 +135,7 @@ def test_stream_extreme_pixel(ca, cuda, dims, ws, C, kind, which, value, first):
     no row's scores all grow with it beyond some 10^3 (a row's log-sum-exp is
     kept in Float32)."""
     sim = ca.DistanceSimilarity() if kind else ca.DotSimilarity()
+    assert min(routes(dims, ws, C, 1, 1, kind, False)) >= 22
     shape = shape_of(dims, C, 1)
     at = tuple(n // 32 * 16 + (0 if first else 5) for n in reversed(dims))
     xs = [seeded(60 + i, shape) for i in range(4)]
