@@ -23,11 +23,13 @@
 // {4-11, 16-19, 28-31} and the same plus 32).
 //
 // What bounds it: the matrix values' way through the texture path (each lane
-// its own 16 bytes, some 40 cycles an instruction: 62% busy) and the matrix
-// cores (128 cycles for a block and 16 components).  Workgroups are not
-// persistent: two fit a CU, and one stages while the other walks.  A 200x120
-// image, window 23, 32 components: A x 230 -> 54 us, A' x 282 -> 65 us (51 MB of
-// values, 10 us at the rate of a large copy).
+// its own 16 bytes, some 40 cycles an instruction) and the wait for it.  A 200x120
+// image, window 23, 32 components: A x 230 -> 53 us, A' x 282 -> 65 us (51 MB of
+// values, 10 us at the rate of a large copy) in 1.5 wavefronts a SIMD, the
+// texture path's data side 0.52 of the time busy, its addresses 0.3, the matrix
+// cores 0.16 (128 cycles for a block and 16 components), and 73 / 88 MB read from
+// memory.  Workgroups are not persistent: two fit a CU, and one stages while the
+// other walks.
 //
 // Values outside a window count as 0 but meet x in the product, so a result
 // that is not a number is formed again from its own window alone.
@@ -535,28 +537,37 @@ hipError_t launch_two(const MxPlan &pl, const MxArgs &f, const MxArgs &t, hipStr
 }  // namespace
 
 // Where these kernels run; elsewhere the row, band and wide kernels do.
-// Measured both ways (us, others -> these: A x / A' x / the pullback's pair),
-// images of 68x60 to 256x254 with 1 to 4 units, 8 to 64 components:
-//  - windows past 15: 68x60, ws 17, 32 components 216/256/259 -> 23/29/29;
-//    4 x 128x126, ws 25, 251/303/329 -> 112/94/195.  The band kernels (to 31) pass
-//    once over each row of A, these fetch its lines some three times: with
-//    more values than the last-level cache holds (256 MB) that costs more than
-//    the products (4 x 256x254, ws 25: 358/416/758 against 417/389/683, ws 31:
-//    458/505/932 against 777/702/1313; ws 21, 115 M values, still
-//    300/373/638 -> 291/287/519).
+// Measured both ways (us, others -> these: A x / A' x / the pullback's pair):
+//  - windows past 15.  The band kernels (to 31) leave the chip idle on few pixels,
+//    some 9 us a window column however few, and pass once over each row of A,
+//    where these fetch its lines some three times: 2.0 to 3.7 us for a million
+//    values, rising with the window, against 3.2 (ws 17) falling to 1.8 (ws 31),
+//    twice that for more than 32 components.  200x120, 32 components, ws 17 179/222/224 ->
+//    30/38/63, ws 31 295/361/359 -> 105/106/175; 4 x 256x254, 32 components, ws 21 (115 M
+//    values) 301/332/584 -> 297/277/486, ws 23 (138 M) 325/359/629 against 384/365/657,
+//    ws 31 444/475/870 against 757/646/1206, 64 components, ws 25 (163 M) 612/709/1264 ->
+//    511/514/904, ws 31 766/840/1569 against 914/869/1606; 2 units, ws 25, 32 components
+//    (81 M) 251/304/358 -> 244/216/367, ws 29 (109 M) 284/346/429 against 398/253/544, ws 31
+//    (125 M) 305/366/459 against 473/319/664; 8 x 200x120, ws 23 (102 M) 338/405/657 ->
+//    312/295/515.
 //  - windows 7 to 15 with few components and pixels, where the row kernels
-//    leave matrix cores or CUs idle: 128x126, 16 components, ws 7 13/14/16 ->
-//    11/13/16, ws 13 27/29/32 -> 14/17/21; with 32 components ws 11 17/18/29
-//    against 16/19/25, with 4 units 15/16/23 against 17/20/31.
+//    leave matrix cores or CUs idle: 128x126, 16 components, ws 7 13/13/14 ->
+//    11/12/15, ws 13 27/29/32 -> 14/17/21; 2 units, ws 7 14/15/15 -> 13/15/20 (its pair
+//    stays), ws 9 19/19/20 -> 11/15/20, ws 11 23/25/26 -> 17/20/27; with 24 components ws 11
+//    17/18/25 against 16/19/23, 2 units 17/19/26 against 21/23/33; 256x254, 16
+//    components, ws 9 19/20/26 against 15/20/35, ws 11 24/26/33 against 24/27/47.
 //  - lines from ws 15 on: 65536, ws 15, 32 components 19/24/52 -> 9/10/18; 8 x
 //    65536, ws 63, 64 components 169/184/363 -> 116/126/275; under that 8
 //    components of 8 x 65536 at ws 7 take 22/23/58 against 29/32/72.
 bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb, int products) {
-    const int64_t px = g.P * nb;
-    if (g.nsp == 1 ? g.ws < 15
-                   : g.ws < 7 || (g.ws <= 15 ? (int64_t)C * ncomp > 16 || px > (1 << 15)
-                                             : g.ws <= 31 && px * g.K > 120000000))
-        return false;
+    const int64_t px = g.P * nb, values = px * g.K, ncr = (int64_t)C * ncomp;
+    if (g.nsp == 1) {
+        if (g.ws < 15) return false;
+    } else if (g.ws <= 15) {
+        if (g.ws < (products == 2 ? 9 : 7) || ncr > 16 || px > (1 << 15)) return false;
+    } else if (g.ws <= 31) {
+        if (values > (g.ws > 25 ? 75000000 : ncr > 32 ? 170000000 : 120000000)) return false;
+    }
     return mx_plan(g, C, ncomp, nb, products).ok;
 }
 

@@ -12,10 +12,9 @@
 // and stored in 16-byte pieces (a lane's four scores stored as they lie would
 // take the texture path 40 cycles for each 16 bytes a lane).
 //
-// What bounds it: dot products by issue (matrix cores a third of the time, the
-// vector instructions of staging and of the rows' assembly a fifth), differences
-// by LDS: a 16-byte read for 8 vector instructions, or 16 where a wavefront
-// takes two query blocks.  200x120, window 23, 32 components: 171 -> 48 us,
+// What bounds it: issue.  Distance at 200x120, window 23, 32 components: vector
+// instructions 0.82 of the time, LDS 0.42 (a 16-byte read for 8 vector instructions,
+// or 16 where a wavefront takes two query blocks), stores at 0.7 TB/s.  200x120, window 23, 32 components: 171 -> 48 us,
 // Distance 213 -> 73 us (51 MB of scores, 10 us at the rate of a large copy).
 #include <algorithm>
 
@@ -392,11 +391,14 @@ hipError_t launch_kind(const SimPlan &pl, hipStream_t s) {
 // against 145) and the sub-row kernel (lines, wider windows).  Measured both ways
 // (us, sub-row kernel -> this one, dot / Distance): 68x60, ws 17, 32 components
 // 119/154 -> 18/36; 200x120, ws 23, 171/213 -> 48/73; 4 x 256x254, ws 17, 434/480 ->
-// 159/282, ws 31 1294/1338 -> 575/954, with 64 components 1500/1674 -> 845/1620;
-// more components cost the differences 21 us each there against 10 (2 x 128x126: 3
-// against 6), so large images of those keep the sub-row kernel.
+// 159/282, ws 31 1294/1338 -> 575/954, 64 components 1488/1670 -> 844/1627.  Past
+// 64 components the differences of windows 27 to 31 on large images stay: 4 x 256x254,
+// ws 31, 72 components 1781 against 1806, 96 2164 against 2293; 2 units, ws 27, 72
+// components 727 against 717, 96 860 against 900, ws 31 916 against 918 and 1068 against
+// 1160; one unit (65024 pixels), ws 31, 72 689 -> 476; ws 33, 2 units, 72 components
+// 1169 -> 920.
 bool sim_mx_supported(bool dist, const Geom &g, int C, int ncomp, int64_t nb) {
-    if (g.ws <= 15 || (dist && g.ws > 25 && (int64_t)C * ncomp > 64 && g.P * nb > 100000)) return false;
+    if (g.ws <= 15 || (dist && g.ws > 25 && g.ws < 33 && (int64_t)C * ncomp > 64 && g.P * nb > 100000)) return false;
     return sim_best(dist, g, C, ncomp, nb).ok;
 }
 
