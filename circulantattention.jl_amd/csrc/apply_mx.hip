@@ -35,6 +35,7 @@
 // that is not a number is formed again from its own window alone.
 #include <algorithm>
 
+#include "buffer_dma.h"
 #include "circatt_common.h"
 #include "circatt_kernels.h"
 
@@ -44,11 +45,13 @@ namespace circatt {
 namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
-typedef int i4v __attribute__((ext_vector_type(4)));
-constexpr unsigned kRsrcWord3 = 0x00020000;  // raw buffer, 32-bit data
-// byte offset past every buffer (buffers are shorter): loads from there give 0
-constexpr int kOut = 0x7fffff00;
-constexpr int64_t kMaxBytes = 0x7ffffe00;
+using dma::dma16;
+using dma::dma_rsrc;
+using dma::i4v;
+using dma::kMaxBytes;
+using dma::kOut;
+using dma::rsrc;
+using dma::wrap;
 // Matrix values are fetched in bursts of kBurst blocks, a burst ahead of the
 // products: the blocks of a burst lie in the same cache lines (a window row is
 // a third of a line at ws 11), which loads spread over the walk would fetch
@@ -68,22 +71,6 @@ struct MxArgs {
     FastDiv div_pass, div_tiles, div_th, div_cr;
 };
 
-__device__ __forceinline__ i4v dma_rsrc(const float *p, int bytes) {
-    const uint64_t b = reinterpret_cast<uint64_t>(p);
-    return i4v{(int)(uint32_t)b, (int)((b >> 32) & 0xffffu), bytes, (int)kRsrcWord3};
-}
-// 16-byte LDS-DMA load: each active lane's four floats from byte voff + soff of
-// the buffer to LDS byte m0 + 16 lane.  The caller waits (vmcnt(0) and a
-// barrier).
-__device__ __forceinline__ void dma16(i4v rs, unsigned m0, int voff, int soff) {
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :
-                 : "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0)
-                 : "memory");
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const float *p, int bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0, bytes, kRsrcWord3);
-}
 __device__ __forceinline__ float gsum(float v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
@@ -92,13 +79,6 @@ __device__ __forceinline__ float gsum(float v) {
 // offset of component k from component 0 (floats)
 __device__ __forceinline__ int coff(const MxArgs &a, int k) {
     return a.pm == 2 ? 2 * a.P * (k >> 1) + (k & 1) : a.P * k;
-}
-
-// v mod n for v in [-n, 2 n) (an integer remainder expands into some 35 vector
-// instructions, a dozen of them per block of a wavefront at the border)
-__device__ __forceinline__ int wrap(int v, int n) {
-    v += v < 0 ? n : 0;
-    return v - (v >= n ? n : 0);
 }
 
 // the products of one wavefront's pixels from their own windows alone: lane c

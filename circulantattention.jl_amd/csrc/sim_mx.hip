@@ -18,6 +18,7 @@
 // Distance 213 -> 73 us (51 MB of scores, 10 us at the rate of a large copy).
 #include <algorithm>
 
+#include "buffer_dma.h"
 #include "circatt_common.h"
 #include "circatt_kernels.h"
 
@@ -28,11 +29,13 @@ namespace {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef f4 f4u __attribute__((aligned(4)));
-typedef int i4v __attribute__((ext_vector_type(4)));
-constexpr unsigned kRsrcWord3 = 0x00020000;  // raw buffer, 32-bit data
-// byte offset past every buffer (buffers are shorter): loads from there give 0
-constexpr int kOut = 0x7fffff00;
-constexpr int64_t kMaxBytes = 0x7ffffe00;
+using dma::dma16;
+using dma::dma_rsrc;
+using dma::i4v;
+using dma::kMaxBytes;
+using dma::kOut;
+using dma::rsrc;
+using dma::wrap;
 constexpr int kLds = 160 * 1024;
 constexpr int kNW = 2;               // wavefronts along each dimension of a workgroup
 constexpr int kW = kNW * kNW;
@@ -49,31 +52,9 @@ struct SimArgs {
     FastDiv div_tiles, div_th, div_strip, div_cr;
 };
 
-__device__ __forceinline__ i4v dma_rsrc(const float *p, int bytes) {
-    const uint64_t b = reinterpret_cast<uint64_t>(p);
-    return i4v{(int)(uint32_t)b, (int)((b >> 32) & 0xffffu), bytes, (int)kRsrcWord3};
-}
-// 16-byte LDS-DMA load: each active lane's four floats from byte voff + soff of
-// the buffer to LDS byte m0 + 16 lane.  The caller waits (vmcnt(0) and a
-// barrier).
-__device__ __forceinline__ void dma16(i4v rs, unsigned m0, int voff, int soff) {
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :
-                 : "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0)
-                 : "memory");
-}
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const float *p, int bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0, bytes, kRsrcWord3);
-}
 __device__ __forceinline__ float load(__amdgpu_buffer_rsrc_t r, int o) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0));
 }
-// v mod n for v in [-n, 2 n)
-__device__ __forceinline__ int wrap(int v, int n) {
-    v += v < 0 ? n : 0;
-    return v - (v >= n ? n : 0);
-}
-
 // Block columns of a wavefront: a window to 17 whole, wider ones in strips whose
 // scores leave registers and LDS for 3 or 4 wavefronts per SIMD.
 constexpr int strip_of(int nk) { return nk <= 5 ? nk : nk == 6 ? 3 : 2; }
