@@ -532,8 +532,9 @@ hipError_t launch_two(const MxPlan &pl, const MxArgs &f, const MxArgs &t, hipStr
 //    312/295/515.
 //  - windows 7 to 15 with few components and pixels, where the row kernels
 //    leave matrix cores or CUs idle: 128x126, 16 components, ws 7 13/13/14 ->
-//    11/12/15, ws 13 27/29/32 -> 14/17/21; 2 units, ws 7 14/15/15 -> 13/15/20 (its pair
-//    stays), ws 9 19/19/20 -> 11/15/20, ws 11 23/25/26 -> 17/20/27; with 24 components ws 11
+//    11/12/15, ws 13 27/29/32 -> 14/17/21; 2 units, ws 7 14/15/15 -> 13/15/20 (the pair
+//    slower there, its sums the more precise: 2.5e-7 of 2-norm error in a step at
+//    97x75, 4 units, against 2.7e-7), ws 9 19/19/20 -> 11/15/20, ws 11 23/25/26 -> 17/20/27; with 24 components ws 11
 //    17/18/25 against 16/19/23, 2 units 17/19/26 against 21/23/33; 256x254, 16
 //    components, ws 9 19/20/26 against 15/20/35, ws 11 24/26/33 against 24/27/47.
 //  - lines from ws 15 on: 65536, ws 15, 32 components 19/24/52 -> 9/10/18; 8 x
@@ -544,7 +545,7 @@ bool apply_mx_supported(const Geom &g, int C, int ncomp, int64_t nb, int product
     if (g.nsp == 1) {
         if (g.ws < 15) return false;
     } else if (g.ws <= 15) {
-        if (g.ws < (products == 2 ? 9 : 7) || ncr > 16 || px > (1 << 15)) return false;
+        if (g.ws < 7 || ncr > 16 || px > (1 << 15)) return false;
     } else if (g.ws <= 31) {
         if (values > (g.ws > 25 ? 75000000 : ncr > 32 ? 170000000 : 120000000)) return false;
     }

@@ -40,25 +40,25 @@
 //
 // What bounds it.  On large images the issue of vector and matrix-core
 // instructions, which add up on a SIMD: 512x512, 32 components, Distance, ws 31,
-// forward 0.59 of the time vector and 0.31 matrix-core, query-centric 0.54 and 0.35,
-// key-centric 0.46 and 0.31 and the rest for registers that spill (25 to 80 in the
-// key-centric kernels of 16 wavefronts or 48 and more components with Distance, up
-// to 29 in the query-centric ones of 16; the forward has none).  Images of one round
-// of workgroups are bound by one workgroup's own chain of staging, barriers and
-// walk (0.36 and 0.2 at 2 x 131x101).  Larger tiles stage less per pixel: see the
-// rule at dispatch.  Against the Float32 run-time-window kernels of fused_impl.h
-// (forward / query- / key-centric pass, us): 512x512 as above 720 / 907 / 1115 ->
-// 385 / 495 / 766; 131x101, 48 components, 2 heads, B = 2, ws 9: 179 / 262 / 315 ->
-// 35 / 41 / 51; 128x96, 64 components, B = 2, ws 15: 102 / 127 / 145 -> 47 / 56 / 69; a
-// line of 30011, 64 components, B = 4, ws 31: 124 / 357 / 493 -> 39 / 48 / 56; 150x170, 8
-// components, B = 4, ws 9: 49 / 55 / 70 -> 27 / 31 / 49.  (Halves took 300 / 400 / 567 in the
-// first, 33 / 38 / 46 in the second.)
+// forward 0.57 of the time vector and 0.30 matrix-core, query-centric 0.54 and 0.35,
+// key-centric 0.54 and 0.37.  Images of one round of workgroups are bound by one
+// workgroup's own chain of staging, barriers and walk (0.36 and 0.2 at 2 x 131x101).
+// Some kernels spill registers: none of the forward's; the query-centric ones of 16
+// wavefronts with planar Distance 11; the key-centric ones of 16 wavefronts 5 to 41, and
+// of 48 and 64 components with Distance, or on the 3 x 2 tile, 2 to 49 (512x512 as above
+// writes 47 MB for 35 and 115 for 67).  Larger tiles stage less per pixel: see the rule
+// at dispatch.  Against the Float32 run-time-window kernels of fused_impl.h (forward /
+// query- / key-centric pass, us): 512x512 as above 720 / 911 / 1113 -> 372 / 461 / 579;
+// 131x101, 48 components, 2 heads, B = 2, ws 9: 179 / 263 / 314 -> 35 / 42 / 52; 128x96, 64
+// components, B = 2, ws 15: 103 / 127 / 145 -> 48 / 57 / 69; a line of 30011, 64 components,
+// B = 4, ws 31: 130 / 356 / 494 -> 41 / 48 / 56; 150x170, 8 components, B = 4, ws 9: 50 / 56 /
+// 71 -> 28 / 31 / 40.  (Halves took 311 / 396 / 568 in the first, 33 / 38 / 46 in the second.)
 //
 // Precision.  Relative 2-norm errors against 64 bits on N(0,1) data, y / dq / dk / dv
 // in units of 1e-7, Float32 kernels -> these: 512x512 as above 8.2 / 11.6 / 10.6 / 9.6 ->
 // 5.8 / 8.8 / 7.1 / 6.5; 131x101 2.7 / 3.5 / 3.4 / 3.3 -> 2.2 / 2.7 / 2.6 / 2.5; 8 components,
-// ws 3 0.95 / 1.8 / 1.7 / 1.5 -> 0.84 / 1.5 / 1.5 / 1.2, ws 21 3.2 / 4.6 / 4.3 / 4.2 ->
-// 1.8 / 2.6 / 2.5 / 2.3; smaller at every window and component count measured.
+// ws 3 0.95 / 1.8 / 1.7 / 1.5 -> 0.84 / 1.5 / 1.6 / 1.3, ws 21 3.2 / 4.6 / 4.3 / 4.2 ->
+// 1.8 / 2.6 / 3.9 / 3.8; smaller at every window and component count measured.
 //
 // Range.  Staged tensors carry a factor 2^24 and the register partner of a dP
 // product a power of two per pixel, so that the thirds of small values stay
@@ -285,6 +285,11 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
     constexpr int PXW = 64 / NTP;           // staged pixels per wave task
     constexpr int RB = ONE ? 16 : 4;        // rows of a block
     constexpr bool KV = MODE == BWDKV;
+    // Loads of the next chunk after the walk instead of before it: the backward
+    // passes of 16 wavefronts (128 registers each) would spill 25 to 80 registers
+    // around them (512x512, 32 components, Distance, ws 31, query- / key-centric pass
+    // 480 / 740 -> 461 / 579 us; without Distance 416 / 574 -> 416 / 536; the forward's fit)
+    constexpr bool LATE = MODE != FWD && EU == 4;
     char *const lds = reinterpret_cast<char *>(circatt_lds2);
     float *const cen = reinterpret_cast<float *>(lds + a.oc);
     float *const sc0 = reinterpret_cast<float *>(lds + a.os);
@@ -677,7 +682,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
 
             const bool lastch = ch + 1 == a.nchunk;
             if (lastch && has_next) decode(nitem, xunit, xh0, xw0);
-            load_stage(xunit, xh0, xw0, lastch ? 0 : ch + 1);
+            if constexpr (!LATE) load_stage(xunit, xh0, xw0, lastch ? 0 : ch + 1);
             if constexpr (DIST)
                 nmu = load_centre(xunit, xh0, xw0);
 
@@ -836,6 +841,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 if (bc < 0 || bc >= (ONE ? 1 : a.nk)) continue;
                 walk(bc, cc);
             }
+            if constexpr (LATE) load_stage(xunit, xh0, xw0, lastch ? 0 : ch + 1);
         }
 
         // ---- results ----
@@ -996,28 +1002,31 @@ hipError_t launch_shape(const Args &a0, const Shape &sh, int nunits, int cus, hi
 template <int NT, int MODE, bool DIST, bool ONE, bool CL>
 hipError_t dispatch(const Args &a, int nunits, int cus, hipStream_t s) {
     // Tiles of 4 x 2 wavefronts; workgroups of these are one a CU in most cases.
-    // us, forward / query- / key-centric pass, at the crossings:
+    // us, forward / query- / key-centric pass, at the crossings (256 CUs):
     //   tiles    shape                      2 x 2          4 x 2         8 x 2
-    //   96       32 components, ws 9        14/16/19       15/17/21
-    //            64, ws 15                  40/44/54       44/51/63
-    //   144      32, ws 9                   16/19/22       16/17/22
-    //            64, ws 15                  70/79/98       44/52/63
-    //   256      32, ws 17                  31/37/45       25/31/39      34/42/64
-    //   288      32, ws 9                   25/29/34       27/32/39      21/26/41
-    //            32, ws 31, Distance        136/156/185    149/173/204   96/122/180
-    //   512      32, ws 17                  56/66/83       45/55/69      38/48/78
-    //            32, ws 31, Distance        165/187/225    153/178/208   101/136/202
-    //   544      32, ws 17                  69/83/103      64/79/98      67/85/133
-    //   1536     32, ws 17                  155/188/234    126/153/193   102/130/210
-    //            32, ws 31, Distance        471/543/654    450/522/615   283/371/572
-    // (8 x 2 in the key-centric pass spills registers, which narrow windows repay less)
+    //   96       32 components, ws 9        14/15/19       15/17/21      20/22/28
+    //            64, ws 15                  40/44/54       44/50/63
+    //   144      32, ws 9                   16/19/23       15/17/22      20/22/28
+    //            64, ws 15                  70/79/96       44/52/64
+    //   256      32, ws 17                  30/35/44       25/30/38      34/39/51
+    //   288      32, ws 9                   24/28/34       26/31/39      21/24/30
+    //            32, ws 31, Distance        134/150/183    146/167/205   93/115/142
+    //   512      16, ws 9                   21/23/28       20/23/28      16/18/23
+    //            32, ws 17                  55/66/84       46/55/69      38/45/59
+    //            32, ws 31, Distance        161/184/227    146/169/209   94/121/154
+    //   544      32, ws 17                  69/82/103      64/78/98      68/79/104
+    //            32, ws 31, Distance        206/229/279    213/247/306   182/225/283
+    //   768      32, ws 17                  80/95/121      66/78/99      69/79/105
+    //   1200     32, ws 9                   56/66/80       59/69/86      57/67/85
+    //   1536     32, ws 17                  154/184/235    125/152/194   102/120/158
+    //            32, ws 31, Distance        463/529/654    438/502/618   270/344/436
     const int64_t tiles = (int64_t)(ONE ? (a.n1 + 127) / 128 : ((a.n1 + 15) / 16) * ((a.n2 + 7) / 8)) * nunits;
     if constexpr (NT <= 2 && !ONE) {
         // twice the tile where that saves rounds of workgroups: a round of these
         // takes some one and a half times as long
         const Shape b = shape_of<NT, 8, 2, 1, DIST, MODE, ONE>(a.p);
         const int64_t r8 = (tiles + 2 * cus - 1) / (2 * cus), r4 = (tiles + cus - 1) / cus;
-        if (b.ok && 3 * r8 < 2 * r4 && (MODE != BWDKV || a.p >= 11))
+        if (b.ok && 3 * r8 < 2 * r4)
             return launch_shape<NT, 8, 2, 1, 4, DIST, MODE, ONE, CL>(a, b, nunits, cus, s);
     }
     const Shape m = shape_of<NT, 4, 2, 3, DIST, MODE, ONE>(a.p);

@@ -53,11 +53,11 @@ def test_every_line_taken_has_a_plan(route, ws):
 
 
 @pytest.mark.parametrize("n1,n2,ws,C,nb,products,taken", [
-    # both sides of the lines in matrix values (75, 120 and 170 million), and window
-    # 7's pair, which the row kernels keep
+    # both sides of the lines in matrix values (75, 120 and 170 million), in pixels and in
+    # components
     (256, 254, 29, 32, 1, 1, True), (256, 254, 29, 32, 2, 2, False), (256, 254, 31, 64, 4, 1, False),
     (256, 254, 21, 32, 4, 1, True), (256, 254, 23, 32, 4, 1, False), (256, 254, 25, 64, 4, 2, True),
-    (256, 254, 33, 32, 4, 1, True), (128, 126, 7, 16, 1, 1, True), (128, 126, 7, 16, 1, 2, False),
+    (256, 254, 33, 32, 4, 1, True), (128, 126, 7, 16, 1, 1, True), (128, 126, 7, 16, 1, 2, True),
     (128, 126, 9, 16, 1, 2, True), (128, 126, 9, 17, 1, 1, False), (200, 180, 9, 16, 1, 1, False),
     (40, 40, 5, 8, 1, 1, False)])
 def test_lines_of_the_rule(route, n1, n2, ws, C, nb, products, taken):

@@ -59,10 +59,10 @@ CASES = [
 # (..., workgroup shapes of the three passes)
 SHAPE_CASES = [
     ((150, 130), 9, 32, 2, 2, 0, False, (42, 42, 42)), ((20000,), 31, 17, 1, 1, 1, False, (42, 42, 42)),
-    ((200, 190), 9, 32, 1, 1, 0, False, (82, 82, 42)), ((200, 190), 21, 16, 1, 1, 0, False, (82, 82, 42)),
-    ((272, 260), 9, 16, 2, 1, 1, False, (82, 82, 42)), ((200, 190), 17, 8, 1, 1, 0, True, (82, 82, 42)),
+    ((200, 190), 9, 32, 1, 1, 0, False, (82, 82, 82)), ((200, 190), 21, 16, 1, 1, 0, False, (82, 82, 82)),
+    ((272, 260), 9, 16, 2, 1, 1, False, (82, 82, 82)), ((200, 190), 17, 8, 1, 1, 0, True, (82, 82, 82)),
     ((193, 190), 23, 32, 1, 1, 0, False, (82, 82, 82)), ((200, 187), 23, 16, 1, 1, 1, True, (82, 82, 82)),
-    ((256, 250), 15, 32, 1, 1, 0, False, (82, 82, 42)),  # window 15: past the Float32 tiles' one round
+    ((256, 250), 15, 32, 1, 1, 0, False, (82, 82, 82)),  # window 15: past the Float32 tiles' one round
     ((40, 30), 31, 64, 1, 1, 1, False, (32, 32, 32)), ((500,), 63, 64, 1, 1, 0, False, (42, 42, 32)),
 ]
 
