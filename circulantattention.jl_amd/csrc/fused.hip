@@ -159,15 +159,19 @@ bool takes_f2d(FusedMode mode, const FusedProblem &pr) {
     if (pr.g.nsp == 1)
         return split && f2h::supported1(pr.g.p, ncr) && pr.g.P * ncr * 4 < (int64_t)INT32_MAX;
     if (!f2d::supported(pr.g.nsp, pr.g.p, ncr, pr.g.P)) return false;
-    // Window 15 at 32 real components on at least as many 16x16 tiles as CUs: the
-    // streamed kernels (launch_stream), whose 32x8 tiles then fill the CUs as well.
-    // us, forward / backward, Float32 tiles -> streamed, Dot: 128x127 16/40 -> 27/68,
-    // 192x192 38/101 -> 36/114, 256x254 57/146 -> 39/122, 320x320 87/232 -> 70/217, 4 x
-    // 256x254 217/567 -> 140/442; Distance: 192x192 40/107 -> 45/139, 256x254 60/154 ->
-    // 48/151, 320x320 92/248 -> 87/268, 4 x 256x254 232/605 -> 176/546.  Complex components,
-    // whose planar loads are half as wide, stay: 256x254 46/127 against 46/136, 4 units
-    // 172/490 against 164/488, Distance 188/524 against 199/582.
-    return !(split && ncr == 32 && pr.g.p == 7 && pr.ncomp == 1 && tiles_of(pr, 16) >= device_cus());
+    // Window 15 at 32 real components: the streamed kernels (launch_stream), whose
+    // errors in the gradients are a quarter of the Float32 tiles' (2.1e-7 against
+    // 8.4e-7), from about where their 32x8 tiles and the 16x16 ones fill the CUs once,
+    // a little later for complex components, whose planar loads are half as wide.  us,
+    // forward / backward, Float32 tiles -> streamed, Dot, Distance: 208x208 (169 tiles of
+    // 16x16) 38/102 -> 38/99, 41/108 -> 46/126; 224x224 (196) 49/131 -> 39/102, 53/141 ->
+    // 47/129; 256x254 57/146 -> 40/113, 61/154 -> 48/145; 272x256 59/161 -> 68/184, 64/173 ->
+    // 85/218; 320x320 87/236 -> 73/192, 91/250 -> 89/244; 4 x 256x254 221/567 -> 149/401,
+    // 232/602 -> 178/496; complex: 208x208 34/96 -> 46/115, 37/104 -> 55/141; 240x240 (225)
+    // 45/126 -> 47/120, 49/135 -> 56/146; 320x320 77/219 -> 87/221, 84/234 -> 104/273; 4 x
+    // 256x254 173/489 -> 168/441, 188/523 -> 201/532.
+    return !(split && ncr == 32 && pr.g.p == 7 &&
+             10 * tiles_of(pr, 16) >= (pr.ncomp == 2 ? 9 : 7) * device_cus());
 }
 
 hipError_t launch_f2d(FusedMode mode, const FusedProblem &pr, hipStream_t s) {
@@ -232,20 +236,19 @@ hipError_t launch_stream(FusedMode mode, const FusedProblem &pr, hipStream_t s, 
         pr.g.p < 1 || pr.g.P * (pr.cl ? all : ncr) * 4 >= (int64_t)fst::kMaxBytes || (pr.cl && ncr % 4 != 0))
         return hipErrorNotSupported;
     const int nt = (ncr + 15) / 16;
-    // Any window and component count, with these exceptions: images of at most one
-    // 8x8 tile of the Float32 kernels a CU, at windows whose 4x4 blocks reach furthest
-    // past them (ws 7: 144 slots for 49, ws 11 and 13: 256 for 121 and 169; window 15 is
-    // compiled into the Float32 kernel of 16 components).  us, forward + backward,
-    // Float32 -> these, 128x127, Dot / Distance, 8 components: ws 3 34 -> 30 / 36 -> 34,
-    // ws 5 34 -> 29 / 37 -> 33, ws 7 37 -> 37 / 39 -> 42, ws 9 46 -> 34 / 53 -> 38, ws 11
-    // 52 -> 52 / 56 -> 60, ws 13 53 -> 52 / 59 -> 60, ws 15 52 -> 68 / 67 -> 78, ws 17 87 ->
-    // 62 / 96 -> 74; 4 complex ones: ws 7 35 -> 41 / 39 -> 46, ws 9 49 -> 40 / 54 -> 48,
-    // ws 13 53 -> 57 / 59 -> 63; 24: ws 7 51 -> 52 / 55 -> 60, ws 11 78 -> 67 / 84 -> 80; 12
-    // complex ones: ws 7 50 -> 58 / 55 -> 68, ws 13 87 -> 74 / 93 -> 88.  Two units of
-    // that size: 8 components, ws 7 50 -> 47 / 53 -> 53, ws 13 72 -> 52 / 78 -> 60, ws 15
-    // 70 -> 72 / 91 -> 84; 24, ws 7 72 -> 61 / 79 -> 71.
-    if (pr.g.nsp == 2 && ((nt <= 2 && pr.g.ws == 7) || (nt == 1 && pr.g.ws >= 11 && pr.g.ws <= 15)) &&
-        tiles_of(pr, 8) <= device_cus())
+    // Any window and component count but one case of the forward: window 15 to 16
+    // components, which is compiled into the Float32 kernel, on up to two of its 8x8
+    // tiles a CU.  us, Float32 -> here, Dot / Distance, 8 components: 128x127 15 -> 19 /
+    // 16 -> 23, 2 units 20 -> 20 / 20 -> 24, 3 units 28 -> 26 / 30 -> 31, 256x254 34 -> 28 /
+    // 36 -> 33; 4 complex ones: 2 units 19 -> 24 / 21 -> 28, 3 units 28 -> 31 / 30 -> 35.
+    // The backward is the more precise here (8 components, ws 13: 2.3e-7 of 2-norm error
+    // in dq against 3.5e-7) and 0.66 to 1.4 times the Float32 kernels' time there.  Other
+    // small images, both passes, 128x127, 8 components: ws 3 34 -> 30 / 36 -> 34, ws 7 37 ->
+    // 39 / 40 -> 41, ws 9 46 -> 34 / 53 -> 38, ws 11 52 -> 52 / 57 -> 60, ws 13 54 -> 53 /
+    // 59 -> 60, ws 17 87 -> 62 / 96 -> 74; 12 complex ones, ws 7 50 -> 58 / 55 -> 68, ws 9
+    // 78 -> 59 / 84 -> 69; three units of that size, ws 7 67 -> 55 / 71 -> 68, ws 13 106 ->
+    // 69 / 116 -> 87.
+    if (mode == MODE_FWD && nt == 1 && pr.g.nsp == 2 && pr.g.ws == 15 && tiles_of(pr, 8) <= 2 * device_cus())
         return hipErrorNotSupported;
     fst::Args a{};
     a.q = pr.q; a.k = pr.k; a.v = pr.v; a.y = pr.y; a.dy = pr.dy; a.lse = pr.lse;

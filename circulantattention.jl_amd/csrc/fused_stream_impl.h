@@ -48,17 +48,20 @@
 // of 48 and 64 components with Distance, or on the 3 x 2 tile, 2 to 49 (512x512 as above
 // writes 47 MB for 35 and 115 for 67).  Larger tiles stage less per pixel: see the rule
 // at dispatch.  Against the Float32 run-time-window kernels of fused_impl.h (forward /
-// query- / key-centric pass, us): 512x512 as above 720 / 911 / 1113 -> 372 / 461 / 579;
-// 131x101, 48 components, 2 heads, B = 2, ws 9: 179 / 263 / 314 -> 35 / 42 / 52; 128x96, 64
-// components, B = 2, ws 15: 103 / 127 / 145 -> 48 / 57 / 69; a line of 30011, 64 components,
-// B = 4, ws 31: 130 / 356 / 494 -> 41 / 48 / 56; 150x170, 8 components, B = 4, ws 9: 50 / 56 /
-// 71 -> 28 / 31 / 40.  (Halves took 311 / 396 / 568 in the first, 33 / 38 / 46 in the second.)
+// query- / key-centric pass, us): 512x512 as above 720 / 911 / 1113 -> 386 / 490 / 623;
+// 131x101, 48 components, 2 heads, B = 2, ws 9: 178 / 263 / 314 -> 36 / 43 / 53; 128x96, 64
+// components, B = 2, ws 15: 104 / 127 / 145 -> 50 / 57 / 70; a line of 30011, 64 components,
+// B = 4, ws 31: 130 / 357 / 493 -> 41 / 48 / 57; 150x170, 8 components, B = 4, ws 9: 49 / 56 /
+// 71 -> 29 / 31 / 41.  (Halves took 311 / 396 / 568 in the first, 33 / 38 / 46 in the second.)
 //
 // Precision.  Relative 2-norm errors against 64 bits on N(0,1) data, y / dq / dk / dv
 // in units of 1e-7, Float32 kernels -> these: 512x512 as above 8.2 / 11.6 / 10.6 / 9.6 ->
-// 5.8 / 8.8 / 7.1 / 6.5; 131x101 2.7 / 3.5 / 3.4 / 3.3 -> 2.2 / 2.7 / 2.6 / 2.5; 8 components,
-// ws 3 0.95 / 1.8 / 1.7 / 1.5 -> 0.84 / 1.5 / 1.6 / 1.3, ws 21 3.2 / 4.6 / 4.3 / 4.2 ->
-// 1.8 / 2.6 / 3.9 / 3.8; smaller at every window and component count measured.
+// 3.7 / 5.7 / 5.3 / 4.7; 131x101 2.7 / 3.5 / 3.4 / 3.3 -> 1.6 / 2.2 / 2.2 / 2.0; 8 components,
+// ws 3 0.95 / 1.8 / 1.7 / 1.5 -> 0.87 / 1.6 / 1.5 / 1.3, ws 21 3.2 / 4.6 / 4.3 / 4.2 ->
+// 1.9 / 2.8 / 2.6 / 2.4; smaller at every window and component count measured.  Half of
+// that comes from forming the smaller partial products from 0 and adding them once
+// (into the running sum, 256x254, 32 components, ws 31: 5.2 / 5.5 / 5.3 / 5.3 -> 2.5 / 3.0 /
+// 3.0 / 2.8, for 1 to 4% of the time).
 //
 // Range.  Staged tensors carry a factor 2^24 and the register partner of a dP
 // product a power of two per pixel, so that the thirds of small values stay
@@ -599,14 +602,9 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
             fsd = KV ? __builtin_amdgcn_ldexpf(1.f, sd + kUpP) : 1.f;
             kb = KV && DIST ? -0.5f * a.c2 * sq : 0.f;
         }
-        // (one component group: the smaller partial products in a sum of their own,
-        // a second chain and fewer roundings of the large one)
-        constexpr int NA = NT == 1 && !KV ? 2 : 1;
-        f4 acc0[NA][NT], acc1[NA][NT];
+        f4 acc0[NT], acc1[NT];
 #pragma unroll
-        for (int i = 0; i < NA; ++i)
-#pragma unroll
-            for (int h = 0; h < NT; ++h) acc0[i][h] = acc1[i][h] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < NT; ++h) acc0[h] = acc1[h] = f4{0.f, 0.f, 0.f, 0.f};
         float lsum = 0.f, corr = 0.f;
         int xunit = unit, xh0 = h0, xw0 = w0;
         const int nitem = item_of(k + 1);
@@ -720,8 +718,9 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 for (int G = 0; G < NG; ++G) x = mfmab(t[G], r[G][0], x);
                 return x;
             };
-            // sums of a block pair's pixels, weighted
-            auto apply = [&](const char *R0, const char *R1, const float (&w)[2][4], f4 (&acc)[NA][NT]) __attribute__((always_inline)) {
+            // sums of a block pair's pixels, weighted: the smaller partial products
+            // from 0 again, so that the sum is rounded at its full size twice
+            auto apply = [&](const char *R0, const char *R1, const float (&w)[2][4], f4 (&acc)[NT]) __attribute__((always_inline)) {
                 u4 wa, wb, wc;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -737,13 +736,12 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     const int o = third_off<NT>(h), d = third_step<NT>(h);
                     const u4 c = ldtr2(R0 + o + 2 * d, R1 + o + 2 * d), b = ldtr2(R0 + o + d, R1 + o + d),
                              a_ = ldtr2(R0 + o, R1 + o);
-                    f4 &lo = acc[NA - 1][h], &hi = acc[0][h];
-                    lo = mfmab(c, wa, lo);
-                    lo = mfmab(a_, wc, lo);
-                    lo = mfmab(b, wb, lo);
-                    lo = mfmab(b, wa, lo);
-                    lo = mfmab(a_, wb, lo);
-                    hi = mfmab(a_, wa, hi);
+                    f4 t = mfmab(c, wa, f4{0.f, 0.f, 0.f, 0.f});
+                    t = mfmab(a_, wc, t);
+                    t = mfmab(b, wb, t);
+                    t = mfmab(b, wa, t);
+                    t = mfmab(a_, wb, t);
+                    acc[h] = mfmab(a_, wa, acc[h] + t);
                 }
             };
             auto walk = [&](int bc, int cc) __attribute__((always_inline)) {
@@ -797,9 +795,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                             m = mx;
                             lsum *= f;
 #pragma unroll
-                            for (int i = 0; i < NA; ++i)
-#pragma unroll
-                                for (int h = 0; h < NT; ++h) acc0[i][h] = acc0[i][h] * f4{f, f, f, f};
+                            for (int h = 0; h < NT; ++h) acc0[h] = acc0[h] * f4{f, f, f, f};
 #pragma unroll
                             for (int u = 0; u < 2; ++u) x[u] = x[u] - f4{mx, mx, mx, mx};
                             ps = probs();
@@ -856,7 +852,6 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                     if (comp_ok(h, 4 * g + r)) o[pm * rpix + coff(c) + coff(r)] = x[r];
             }
         };
-        if constexpr (NA == 2) acc0[0][0] = acc0[0][0] + acc0[1][0];
         // a result that is not finite (values outside the pixel's window, or the
         // powers of two, may have made it so): NaN marks the wavefront's pixels for
         // the second pass below
@@ -866,8 +861,8 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
         for (int h = 0; h < NT; ++h)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                bad |= !(fabsf(acc0[0][h][r]) < INFINITY);
-                if constexpr (KV) bad |= !(fabsf(acc1[0][h][r]) < INFINITY);
+                bad |= !(fabsf(acc0[h][r]) < INFINITY);
+                if constexpr (KV) bad |= !(fabsf(acc1[h][r]) < INFINITY);
             }
         const float l = MODE == FWD ? gsum(lsum) : 1.f;
         const float cs = DIST && MODE != FWD ? gsum(corr) : 0.f;
@@ -882,7 +877,7 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 for (int h = 0; h < NT; ++h) {
                     float x[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_ldexpf(acc0[0][h][r] * inv, -kUp);
+                    for (int r = 0; r < 4; ++r) x[r] = __builtin_amdgcn_ldexpf(acc0[h][r] * inv, -kUp);
                     put4(a.yout, h, x);
                 }
                 if (g == 0) a.lse_out[soff + rpix] = lse_of(m, l, DIST ? 0.5f * sq * a.scale : 0.f);
@@ -894,14 +889,14 @@ __global__ __launch_bounds__(64 * NWH * NWW, EU) void kernel_stream(Args a) {
                 float xk[4], xv[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = __builtin_amdgcn_ldexpf(acc0[0][h][r], -(sd + kUpP + kUp) - a.pe);
+                    float v = __builtin_amdgcn_ldexpf(acc0[h][r], -(sd + kUpP + kUp) - a.pe);
                     if constexpr (DIST) {
                         const float reg = load1(KV ? a.k : a.q, uoff, len, rpix, h, 4 * g + r) -
                                           __shfl(cmu, 16 * h + 4 * g + r);
                         v -= __builtin_amdgcn_ldexpf(cs, -(sd + kUpP) - a.pe) * reg;
                     }
                     xk[r] = v * f;
-                    if constexpr (KV) xv[r] = __builtin_amdgcn_ldexpf(acc1[0][h][r], -kUp - a.pe);
+                    if constexpr (KV) xv[r] = __builtin_amdgcn_ldexpf(acc1[h][r], -kUp - a.pe);
                 }
                 if (rvalid) {
                     put4(KV ? a.dk : a.dq, h, xk);

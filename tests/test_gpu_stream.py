@@ -63,6 +63,7 @@ SHAPE_CASES = [
     ((272, 260), 9, 16, 2, 1, 1, False, (82, 82, 82)), ((200, 190), 17, 8, 1, 1, 0, True, (82, 82, 82)),
     ((193, 190), 23, 32, 1, 1, 0, False, (82, 82, 82)), ((200, 187), 23, 16, 1, 1, 1, True, (82, 82, 82)),
     ((256, 250), 15, 32, 1, 1, 0, False, (82, 82, 82)),  # window 15: past the Float32 tiles' one round
+    ((250, 245), 15, 16, 1, 1, 0, True, (82, 82, 82)), ((40, 36), 15, 8, 1, 1, 0, False, (0, 22, 22)),
     ((40, 30), 31, 64, 1, 1, 1, False, (32, 32, 32)), ((500,), 63, 64, 1, 1, 0, False, (42, 42, 32)),
 ]
 
