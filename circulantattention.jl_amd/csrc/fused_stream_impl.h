@@ -1020,7 +1020,8 @@ hipError_t dispatch(const Args &a, int nunits, int cus, hipStream_t s) {
         // twice the tile where that saves rounds of workgroups: a round of these
         // takes some one and a half times as long
         const Shape b = shape_of<NT, 8, 2, 1, DIST, MODE, ONE>(a.p);
-        const int64_t r8 = (tiles + 2 * cus - 1) / (2 * cus), r4 = (tiles + cus - 1) / cus;
+        const int64_t tall = (int64_t)((a.n1 + 31) / 32) * ((a.n2 + 7) / 8) * nunits;
+        const int64_t r8 = (tall + cus - 1) / cus, r4 = (tiles + cus - 1) / cus;
         if (b.ok && 3 * r8 < 2 * r4)
             return launch_shape<NT, 8, 2, 1, 4, DIST, MODE, ONE, CL>(a, b, nunits, cus, s);
     }

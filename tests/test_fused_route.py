@@ -30,7 +30,9 @@ def route():
     # 2 x 2 wavefronts to half a round of 4 x 2, 8 x 2 where they save rounds
     (dict(n1=128, n2=128, ws=17, dh=32), (22, 22, 22)), (dict(n1=128, n2=136, ws=17, dh=32), (42, 42, 42)),
     (dict(n1=256, n2=128, ws=17, dh=32), (42, 42, 42)), (dict(n1=272, n2=128, ws=17, dh=32), (82, 82, 82)),
-    (dict(n1=256, n2=264, ws=17, dh=32), (42, 42, 42)), (dict(n1=272, n2=128, ws=17, dh=48), (42, 42, 42)),
+    (dict(n1=256, n2=264, ws=17, dh=32), (42, 42, 42)),
+    # (504 tiles of 16x8, but 264 of 32x8)
+    (dict(n1=327, n2=94, ws=23, dh=8, units=2), (42, 42, 42)), (dict(n1=272, n2=128, ws=17, dh=48), (42, 42, 42)),
     # LDS: 64 components from some window on by 3 x 2, past 33 not at all
     (dict(n1=512, n2=512, ws=23, dh=64), (42, 42, 42)), (dict(n1=512, n2=512, ws=31, dh=64), (32, 32, 32)),
     (dict(n1=512, n2=512, ws=35, dh=64), (0, 0, 0)), (dict(n1=512, n2=512, ws=77, dh=32, kind=1), (42, 42, 42)),
